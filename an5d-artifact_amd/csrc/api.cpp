@@ -36,6 +36,13 @@ int hip_fail(hipError_t e, const char* what) {
   void register_variants_##id##_0(std::vector<Variant>&);     \
   void register_variants_##id##_1(std::vector<Variant>&);
 AN5D_STENCILS(AN5D_DECL_REG)
+// cols_inst.hip
+void register_cols_17_0(std::vector<Variant>&);
+void register_cols_17_1(std::vector<Variant>&);
+void register_cols_18_0(std::vector<Variant>&);
+void register_cols_18_1(std::vector<Variant>&);
+void register_cols_19_0(std::vector<Variant>&);
+void register_cols_19_1(std::vector<Variant>&);
 
 std::vector<Variant>& registry() {
   static std::vector<Variant> v = [] {
@@ -44,6 +51,13 @@ std::vector<Variant>& registry() {
   register_variants_##id##_0(out);                            \
   register_variants_##id##_1(out);
     AN5D_STENCILS(AN5D_CALL_REG)
+    // after the others, so the indices of those stay put
+    register_cols_17_0(out);
+    register_cols_17_1(out);
+    register_cols_18_0(out);
+    register_cols_18_1(out);
+    register_cols_19_0(out);
+    register_cols_19_1(out);
     return out;
   }();
   return v;
@@ -135,6 +149,24 @@ int device_cus() {
 // leave most SIMDs idle); without a device to ask, about 8192 wave tiles.
 int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long ntj, int mode) {
   const long long n0 = g.D0 - 2 * g.r;
+  if (v.kind == kCols) {
+    // ntk: workgroups per segment.  A workgroup is one wave per SIMD; a CU with
+    // b of them takes about max(2.4, b) times a lone wave's issue time (fewer
+    // than 2.4 waves leave latency exposed), and a segment costs sl planes plus
+    // half a plane's issue for the warm-up loads.  Fitted to sweeps of sl at
+    // 64^3 .. 512^3 of every stencil and dtype: within 5 % of the best.  At
+    // most 32 planes: longer segments lose the rows their neighbours share in
+    // L2 (box3d2r FP64 512^3: 1386 us at 32, 1527 at 128).
+    const double cus = device_cus() > 0 ? device_cus() : 256;
+    long long best = 1;
+    double best_t = 1e300;
+    for (long long sl = 1; sl <= n0 && sl <= 32; sl++) {
+      const double b = ceil(ntk * cdiv(n0, sl) / cus);
+      const double t = (sl + 0.5) * (b > 2.4 ? b : 2.4);
+      if (t < best_t) { best_t = t; best = sl; }
+    }
+    return (int)best;
+  }
   const bool tiles3 = (v.kind == kSweep || v.kind == kPlane) && g.dim == 3;
   long long slots = 0;
   if ((v.kind == kSweep || v.kind == kPlane || v.kind == kRows) && bt >= 1 && bt <= kMaxBT && v.occ[bt]) {
@@ -175,6 +207,20 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     lp.grid = dim3((unsigned)cdiv(total, 256));
     a.ntk = a.ntj = a.nseg = a.sl = a.SK = a.SJ = 0;
     if (cdiv(total, 256) >= (1LL << 31)) { err = "grid too large"; return false; }
+    return true;
+  }
+  if (v.kind == kCols) {
+    // lanes of ck cells over the plane, row-major, in blocks of 256 per segment
+    const long long ntk = cdiv(nk, v.ck), nblk = cdiv(ntk * nj, 256);
+    if (nk < v.ck) { err = "rows shorter than a lane's run"; return false; }
+    if (ntk * nj >= (1LL << 30)) { err = "grid too large"; return false; }
+    if (sl <= 0) sl = default_sl(v, bt, g, nblk, 1, mode);
+    const long long nseg = cdiv(n0, sl);
+    a.ntk = (int)ntk; a.ntj = (int)nblk; a.nseg = (int)nseg; a.sl = sl;
+    a.SK = v.ck; a.SJ = 1;
+    lp.block = dim3(256);
+    if (nblk * nseg >= (1LL << 31)) { err = "grid too large"; return false; }
+    lp.grid = dim3((unsigned)(nblk * nseg));
     return true;
   }
   if (v.kind == kPlane) {
@@ -275,6 +321,26 @@ bool build_coefs(const an5d_problem* p, std::vector<unsigned char>& bytes, int& 
     memcpy(&bytes[(nt + 1) * 4], &rc, 4);
   }
   return true;
+}
+
+// The column kernel's order of the table build_coefs made: the centre taps by
+// plane, then for every row d1 the (2r+1) x (2r+1) block [plane d0][d2] (the
+// centre's place is there and not read), then the divisor and its reciprocal
+// as before.  The taps' signs go into the values (a - c*v == a + (-c)*v); the
+// fast mode's table has them already.
+void cols_coefs(const an5d_problem* p, std::vector<unsigned char>& bytes, int mode) {
+  const StencilRT& s = stencil_rt(p->stencil);
+  const size_t esz = p->dtype == AN5D_FLOAT64 ? 8 : 4;
+  const int r = s.rad, w = 2 * r + 1;
+  std::vector<unsigned char> out((size_t)(w + w * w * w + 2) * esz, 0);
+  for (int q = 0; q < s.ntaps; q++) {
+    const TapDef& t = s.taps[q];
+    const int slot = t.d1 == 0 && t.d2 == 0 ? t.d0 + r : w + ((t.d1 + r) * w + t.d0 + r) * w + t.d2 + r;
+    memcpy(&out[slot * esz], &bytes[q * esz], esz);
+    if (t.sign < 0 && mode != AN5D_FAST) out[slot * esz + esz - 1] ^= 0x80;  // little-endian sign bit
+  }
+  memcpy(&out[out.size() - 2 * esz], &bytes[s.ntaps * esz], 2 * esz);
+  bytes.swap(out);
 }
 
 // The shared-product form applies when the stencil is a radius-1 star (a
@@ -386,6 +452,16 @@ int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout,
       if (sl == 0) sl = tc.sl;
     } else {
       v = vs[0];  // first sweep shape, or the direct kernel when none exists
+    }
+  }
+  // a table row of a like size may not fit this grid's extents
+  if (want_v < 0 && v->kind == kCols) {
+    Geom g;
+    LaunchPlan lp;
+    std::string err;
+    if (!make_geom(p, g, err) || !plan_launch(*v, 1, g, sl, lp, err, mode)) {
+      v = vs[0];
+      sl = cfg ? cfg->sl : 0;
     }
   }
   int bt = want_bt ? want_bt : default_bt(s, p->dtype);
@@ -543,6 +619,7 @@ int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout,
     if (share && v->fn_share[k] && v->share_scratch[k] && v->share_scratch[k]() == 0) return kLaunchShare;
     return rcfg.mode;
   };
+  if (v->kind == kCols) cols_coefs(p, cbytes, rcfg.mode);
   const void* dcoef = nullptr;
   rc = device_coefs(cbytes, &dcoef);
   if (rc) return rc;

@@ -116,7 +116,7 @@ double ops_per_update(const StencilRT& s, const Variant& v, int mode, bool has_d
     if (s.dim == 3) ops += 2.0 * s.rad * 2.0 / v.cj;
   } else if (v.kind == kPlane) {
     ops += 2.0 * s.rad;  // the dim-0 queue shifts by one plane per step
-  } else {
+  } else if (v.kind != kCols) {
     ops += 0.5 * s.ntaps;  // address arithmetic of the direct kernel
   }
   return ops;
@@ -141,6 +141,9 @@ double model_gstencil(const an5d_problem* p, const Variant& v, int bt, int sl, i
     if (g.dim == 3) ovj = lp.args.ntj * (double)v.nw * v.cj / nj;
     ovi = (lp.args.nseg * (double)lp.args.sl + 2.0 * bt * g.r * lp.args.nseg) / n0;
     waves = (double)lp.args.ntk * lp.args.ntj * lp.args.nseg * (g.dim == 3 ? v.nw : 1);
+  } else if (v.kind == kCols) {
+    waves = (double)lp.args.ntj * lp.args.nseg * 4;
+    ovi = (lp.args.sl + 0.5 * g.r) / lp.args.sl;
   } else if (v.kind == kPlane) {
     ovk = lp.args.ntk * 64.0 * v.ck / nk;
     ovj = lp.args.ntj * (double)v.nw * v.cj / nj;

@@ -51,6 +51,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
 bool coefs_shareable(const an5d_problem* p, const std::vector<unsigned char>& bytes);
 bool build_coefs(const an5d_problem* p, std::vector<unsigned char>& bytes, int& has_div,
                  double& gscale, std::string& err, int mode = 0);
+void cols_coefs(const an5d_problem* p, std::vector<unsigned char>& bytes, int mode);
 int device_coefs(const std::vector<unsigned char>& bytes, const void** out);
 // The current device's staging grid of at least `bytes`; `hold` keeps other
 // host calls on that device from using or regrowing it until released.

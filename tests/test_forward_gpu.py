@@ -333,3 +333,38 @@ def test_forward_host_from_several_threads():
         ref = a.copy()
         O.run("j2d5pt", ref, n, T)
         assert np.array_equal(o[T % 2], ref[T % 2])
+
+
+@pytest.mark.parametrize("name", ["box3d2r", "box3d3r", "box3d4r"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_box3d_column_kernel_ragged_grids(name, dt):
+    """The column kernel of the wide 3D boxes (kind 4): rows that end inside a
+    lane's run, rows of one run only, a last workgroup that is nearly empty,
+    segments of one plane, of fewer planes than the stencil's and the default;
+    bit for bit the oracle in exact mode (also over a divisor), within 1e-5 /
+    1e-12 of the field's largest value in FMA mode."""
+    v, = [v for v in pyan5d.variants(name, 0 if dt == np.float32 else 1) if v["kind"] == 4]
+    for n, sl, div in [([1, 1, 4], 0, -1.0), ([3, 5, 7], 1, 7.0), ([9, 17, 66], 3, -1.0), ([12, 33, 31], 0, 118.0)]:
+        T = 3
+        print(f"case columns {name} {np.dtype(dt).name} n={n} sl={sl} divisor={div}", flush=True)
+        A = rand_grid(name, n, dt, seed=sum(n))
+        B, C = A.copy(), A.copy()
+        pyan5d.forward_host(name, A, n, T, variant=v["index"], sl=sl, divisor=div)
+        O.run(name, B, n, T, divisor=div)
+        assert same(A[T % 2], B[T % 2])
+        pyan5d.forward_host(name, C, n, T, variant=v["index"], sl=sl, divisor=div, mode=pyan5d.FAST)
+        got, ref = C[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
+        assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
+
+
+def test_box3d_rows_shorter_than_a_run():
+    """Below one run per row the tuned choice does not fit: the default path
+    takes the direct kernel as before."""
+    n, T = [40, 60, 3], 2
+    print("case columns fallback box3d2r", n, flush=True)
+    assert pyan5d.resolve_config("box3d2r", n, np.float64)["variant"] == 0
+    A = rand_grid("box3d2r", n, np.float64, seed=5)
+    B = A.copy()
+    pyan5d.forward_host("box3d2r", A, n, T)
+    O.run("box3d2r", B, n, T)
+    assert same(A[T % 2], B[T % 2])
