@@ -77,9 +77,9 @@ int occupancy_sweep(int mode) {
                    : occupancy_once<BT, CK, CJ, NW, true, false, WPE>();
 }
 
-template <int CK>
+template <int CK, bool EXACT>
 hipError_t launch_direct(const LaunchArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t st) {
-  hipLaunchKernelGGL((direct_kernel<SID, T, CK>), grid, block, lds, st, to_args<T>(a));
+  hipLaunchKernelGGL((direct_kernel<SID, T, CK, EXACT>), grid, block, lds, st, to_args<T>(a));
   return hipGetLastError();
 }
 
@@ -285,8 +285,8 @@ void AN5D_CAT(register_variants_, AN5D_SID, AN5D_F64)(std::vector<Variant>& out)
   d.kind = kDirect;
   d.ck = direct_ck<SID, T>(); d.cj = 1; d.nw = 4; d.btmax = 1;
   for (auto& l : d.lds) l = 0;
-  d.fn[1] = &launch_direct<direct_ck<SID, T>()>;
-  d.fn_fast[1] = d.fn[1];
+  d.fn[1] = &launch_direct<direct_ck<SID, T>(), true>;
+  d.fn_fast[1] = &launch_direct<direct_ck<SID, T>(), false>;
   out.push_back(d);
   // radius 2-4 3D stars: one step per launch with the plane staged in LDS
   if constexpr (plane_taps_ok<Def<SID>>() && Def<SID>::rad >= 2) {

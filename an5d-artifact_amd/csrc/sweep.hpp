@@ -874,7 +874,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) 
 // One step without temporal blocking: every thread evaluates CK adjacent
 // interior cells straight from global memory.  Used where the register
 // pipeline does not fit (the radius-2..4 3D boxes) and as a baseline.
-template <int ID, typename T, int CK>
+template <int ID, typename T, int CK, bool EXACT>
 __global__ __launch_bounds__(256) void direct_kernel(SweepArgs<T> a) {
   using D = Def<ID>;
   constexpr int R = D::rad;
@@ -901,7 +901,8 @@ __global__ __launch_bounds__(256) void direct_kernel(SweepArgs<T> a) {
     if (k >= a.D2 - R) break;
     const T* p = a.src + base + k;
     MemGet<T> get{p, a.s0, a.s1};
-    a.dst[base + k] = eval_point<D, T>(get, c, c[NT], has_div, a.gscale);
+    if constexpr (EXACT || !D::linear) a.dst[base + k] = eval_point<D, T>(get, c, c[NT], has_div, a.gscale);
+    else a.dst[base + k] = eval_fast<D, T>(get, c);
   }
 }
 

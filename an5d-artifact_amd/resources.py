@@ -64,7 +64,7 @@ FIELDS = {
     "sweep_kernel": ["bt", "ck", "cj", "nw", "exact", "mids", "unr", "share"],
     "sweep_kernel_cap": ["bt", "ck", "cj", "nw", "exact", "waves_per_eu"],
     "plane_kernel": ["bt", "ck", "cj", "nw", "exact"],
-    "direct_kernel": ["ck"],
+    "direct_kernel": ["ck", "exact"],
     "adjoint_kernel": ["bt", "ck", "nw"],
     "rows_kernel": ["ck", "nw", "exact"],
     "rows_kernel_cap": ["ck", "nw", "exact", "waves_per_eu"],

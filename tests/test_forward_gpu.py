@@ -368,3 +368,19 @@ def test_box3d_rows_shorter_than_a_run():
     pyan5d.forward_host("box3d2r", A, n, T)
     O.run("box3d2r", B, n, T)
     assert same(A[T % 2], B[T % 2])
+
+
+@pytest.mark.parametrize("name", ["star2d4r", "box3d2r", "box3d3r"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_direct_kernel_fast_mode_with_subtracted_taps(name, dt):
+    """The FMA table carries the taps' signs, so the direct kernel must not
+    apply them again."""
+    v, = [v for v in pyan5d.variants(name, 0 if dt == np.float32 else 1) if v["kind"] == 1]
+    n, T = ([9, 40] if O.info(name)["dim"] == 2 else [6, 7, 9]), 2
+    print(f"case direct fast {name} {np.dtype(dt).name}", flush=True)
+    A = rand_grid(name, n, dt, seed=8)
+    B = A.copy()
+    pyan5d.forward_host(name, A, n, T, variant=v["index"], mode=pyan5d.FAST)
+    O.run(name, B, n, T)
+    got, ref = A[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
+    assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
