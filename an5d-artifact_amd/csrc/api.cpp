@@ -144,50 +144,53 @@ int device_cus() {
   return n;
 }
 
-// Default segment length along dim 0: as many segments as fill the GPU's
-// resident workgroup slots in one round (a partly filled second round would
-// leave most SIMDs idle); without a device to ask, about 8192 wave tiles.
-int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long ntj, int mode) {
+// Default segment length along dim 0.  The time of a launch is taken as
+//   (planes a segment runs) x max(L, waves per SIMD on the busiest CU)
+// in units of one wave's time per plane: waves share a SIMD's issue, fewer
+// than L of them leave latency exposed, and a segment runs its own planes,
+// the 2*bt*R warm-up planes of the sweeps and what fills whole loop bodies.
+// L and the warm-up were fitted to the times of every segment length 1 .. 128
+// over 256^2 .. 8192^2 and 64^3 .. 384^3 (squares, cubes and ragged
+// rectangles, both dtypes): the choice is 1-3 % off the best in the geometric
+// mean, where "as many segments as fill the resident workgroups in one round,
+// 8*bt*R planes at least" was 1.5-2.1 times off (a 256^2 grid got 16 waves).
+int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long ntj) {
   const long long n0 = g.D0 - 2 * g.r;
-  if (v.kind == kCols) {
-    // ntk: workgroups per segment.  A workgroup is one wave per SIMD; a CU with
-    // b of them takes about max(2.4, b) times a lone wave's issue time (fewer
-    // than 2.4 waves leave latency exposed), and a segment costs sl planes plus
-    // half a plane's issue for the warm-up loads.  Fitted to sweeps of sl at
-    // 64^3 .. 512^3 of every stencil and dtype: within 5 % of the best.  At
-    // most 32 planes: longer segments lose the rows their neighbours share in
-    // L2 (box3d2r FP64 512^3: 1386 us at 32, 1527 at 128).
-    const double cus = device_cus() > 0 ? device_cus() : 256;
-    long long best = 1;
-    double best_t = 1e300;
-    for (long long sl = 1; sl <= n0 && sl <= 32; sl++) {
-      const double b = ceil(ntk * cdiv(n0, sl) / cus);
-      const double t = (sl + 0.5) * (b > 2.4 ? b : 2.4);
-      if (t < best_t) { best_t = t; best = sl; }
+  const long long cus = device_cus() > 0 ? device_cus() : 256;
+  const bool tiles3 = g.dim == 3;     // a segment holds ntk * ntj workgroups, else ntk waves
+  const bool cols = v.kind == kCols;  // 3D: ntk workgroups; 2D: ntk runs of a lane
+  double lat = 1.5, warm = 2.0 * bt * g.r + 1;
+  int body = 1;
+  long long longest = n0;
+  if (cols) {
+    // warm-up planes cost their loads only; longer segments lose the rows that
+    // neighbours share in L2 (box3d2r FP64 512^3: 1386 us at 32, 1527 at 128;
+    // box2d4r FP32 8192^2: 196 us at 16, 214 at 32)
+    lat = 2.4;
+    warm = 0.5;
+    longest = g.dim == 3 ? 32 : 16;
+  } else if (v.kind == kPlane && g.r > 1) {
+    lat = 4;  // every plane waits for the tiles of LDS at a barrier
+  } else if (v.kind == kSweep && g.r <= 2) {
+    body = g.r == 1 && bt * v.cj * v.ck <= 36 ? 6 : 2 * g.r + 1;
+  }
+  double best_t = 1e300;
+  long long best = n0 < longest ? n0 : longest;
+  // every count up to 64, then steps of a sixteenth
+  for (long long nseg = cdiv(n0, longest); nseg <= n0; nseg += 1 + (nseg >= 64 ? nseg / 16 : 0)) {
+    const long long sl = cdiv(n0, nseg);
+    const long long waves = cols && !tiles3 ? cdiv(ntk * nseg, 64) : ntk * nseg;
+    const long long wgs = tiles3 ? ntk * ntj * nseg : cdiv(waves, v.nw);
+    const double share = (double)cdiv(wgs, cus) * v.nw / 4;
+    const double planes = body > 1 ? (double)cdiv(sl + (long long)warm, body) * body : sl + warm;
+    const double t = planes * (share > lat ? share : lat);
+    if (t < best_t) {
+      best_t = t;
+      best = sl;
     }
-    return (int)best;
+    if (share > 8 * lat) break;  // more segments only add warm-up
   }
-  const bool tiles3 = (v.kind == kSweep || v.kind == kPlane) && g.dim == 3;
-  long long slots = 0;
-  if ((v.kind == kSweep || v.kind == kPlane || v.kind == kRows) && bt >= 1 && bt <= kMaxBT && v.occ[bt]) {
-    const int occ = v.occ[bt](mode);
-    const int cus = occ > 0 ? device_cus() : 0;
-    slots = (long long)occ * cus * (tiles3 ? 1 : v.nw);  // workgroups (3D) or waves (2D)
-  }
-  long long nseg;
-  if (slots > 0) {
-    const long long per_seg = tiles3 ? ntk * ntj : ntk;
-    nseg = slots / per_seg > 1 ? slots / per_seg : 1;
-  } else {
-    long long tiles = ntk * ntj * (tiles3 ? v.nw : 1);
-    nseg = cdiv(8192, tiles > 0 ? tiles : 1);
-  }
-  long long sl = cdiv(n0, nseg);
-  long long minsl = 8LL * bt * g.r;
-  if (sl < minsl) sl = minsl;
-  if (sl > n0) sl = n0;
-  if (sl < 1) sl = 1;
-  return (int)sl;
+  return (int)(best < 1 ? 1 : best);
 }
 
 bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp,
@@ -214,7 +217,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     const long long ntk = cdiv(nk, v.ck), nblk = cdiv(ntk * nj, 256);
     if (nk < v.ck) { err = "rows shorter than a lane's run"; return false; }
     if (ntk * nj >= (1LL << 30)) { err = "grid too large"; return false; }
-    if (sl <= 0) sl = default_sl(v, bt, g, nblk, 1, mode);
+    if (sl <= 0) sl = default_sl(v, bt, g, nblk, 1);
     const long long nseg = cdiv(n0, sl);
     a.ntk = (int)ntk; a.ntj = (int)nblk; a.nseg = (int)nseg; a.sl = sl;
     a.SK = v.ck; a.SJ = 1;
@@ -228,7 +231,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     if (g.dim != 3) { err = "the plane kernel is 3D only"; return false; }
     const long long TK = 64LL * v.ck, TJ = (long long)v.nw * v.cj;
     const long long ntk = cdiv(nk, TK), ntj = cdiv(nj, TJ);
-    if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj, mode);
+    if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj);
     const long long nseg = cdiv(n0, sl);
     a.ntk = (int)ntk; a.ntj = (int)ntj; a.nseg = (int)nseg; a.sl = sl;
     a.SK = (int)TK; a.SJ = (int)TJ;
@@ -255,7 +258,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     if (SJ <= 0) { err = "bt too deep for this variant's tile height"; return false; }
     ntj = cdiv(nj, SJ);
   }
-  if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj, mode);
+  if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj);
   const long long nseg = cdiv(n0, sl);
   a.ntk = (int)ntk; a.ntj = (int)ntj; a.nseg = (int)nseg; a.sl = sl;
   a.SK = (int)SK; a.SJ = (int)SJ;

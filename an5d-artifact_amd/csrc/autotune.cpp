@@ -210,7 +210,7 @@ extern "C" int an5d_autotune(const an5d_problem* p, void* dA, const an5d_layout*
   };
   std::vector<Cand> cands;
   const long long n0 = g.D0 - 2 * g.r;
-  const int sls[] = {0, 16, 32, 64, 128, 256};
+  const int sls[] = {0, 4, 8, 16, 32, 64, 128, 256};
   for (int vi = 0; vi < (int)vs.size(); vi++) {
     const Variant& v = *vs[vi];
     for (int bt = 1; bt <= v.btmax; bt++) {

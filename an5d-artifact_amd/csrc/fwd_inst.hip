@@ -54,29 +54,6 @@ int share_scratch_once() {
   return n;
 }
 
-// Resident workgroups per CU (0 if the query fails); computed once, on the
-// first device that asks (every device is a gfx950 with the same resources).
-template <int BT, int CK, int CJ, int NW, bool EXACT, bool SHARE = false, int WPE = 0>
-int occupancy_once() {
-  static const int n = [] {
-    const void* k = reinterpret_cast<const void*>(sweep_fn<BT, CK, CJ, NW, EXACT, false, SHARE, WPE>());
-    const size_t lds = sweep_lds_bytes<SID, T, CK, CJ, NW>(BT);
-    static std::atomic<int> done[kMaxDevices];
-    if (lds > 65536 && lds_opt_in(k, lds, done) != hipSuccess) return 0;
-    int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 64 * NW, lds) != hipSuccess) return 0;
-    return blocks;
-  }();
-  return n;
-}
-template <int BT, int CK, int CJ, int NW, int WPE = 0>
-int occupancy_sweep(int mode) {
-  if constexpr (kShare && WPE == 0)
-    if (mode == 2) return occupancy_once<BT, CK, CJ, NW, true, true>();
-  return mode == 1 ? occupancy_once<BT, CK, CJ, NW, false, false, WPE>()
-                   : occupancy_once<BT, CK, CJ, NW, true, false, WPE>();
-}
-
 template <int CK, bool EXACT>
 hipError_t launch_direct(const LaunchArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t st) {
   hipLaunchKernelGGL((direct_kernel<SID, T, CK, EXACT>), grid, block, lds, st, to_args<T>(a));
@@ -97,24 +74,6 @@ hipError_t launch_plane(const LaunchArgs& a, dim3 grid, dim3 block, size_t lds, 
   return hipGetLastError();
 }
 
-template <int CK, int CJ, int NW, bool EXACT>
-int occupancy_plane_once() {
-  static const int n = [] {
-    const void* k = reinterpret_cast<const void*>(&plane_kernel<SID, T, CK, CJ, NW, EXACT>);
-    constexpr size_t lds = plane_lds_bytes<T, CK, CJ, NW, Def<SID>::rad>();
-    static std::atomic<int> done[kMaxDevices];
-    if (lds > 65536 && lds_opt_in(k, lds, done) != hipSuccess) return 0;
-    int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 64 * NW, lds) != hipSuccess) return 0;
-    return blocks;
-  }();
-  return n;
-}
-template <int CK, int CJ, int NW>
-int occupancy_plane(int mode) {
-  return mode ? occupancy_plane_once<CK, CJ, NW, false>() : occupancy_plane_once<CK, CJ, NW, true>();
-}
-
 template <int CK, bool EXACT, int WPE>
 constexpr auto rows_fn() {
   if constexpr (WPE > 0) return &rows_kernel_cap<SID, T, CK, 4, EXACT, WPE>;
@@ -126,21 +85,6 @@ hipError_t launch_rows(const LaunchArgs& a, dim3 grid, dim3 block, size_t lds, h
   constexpr auto kern = rows_fn<CK, EXACT, WPE>();
   hipLaunchKernelGGL(kern, grid, block, 0, st, to_args<T>(a));
   return hipGetLastError();
-}
-
-template <int CK, bool EXACT, int WPE>
-int occupancy_rows_once() {
-  static const int n = [] {
-    int blocks = 0;
-    const void* k = reinterpret_cast<const void*>(rows_fn<CK, EXACT, WPE>());
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 64 * 4, 0) != hipSuccess) return 0;
-    return blocks;
-  }();
-  return n;
-}
-template <int CK, int WPE>
-int occupancy_rows(int mode) {
-  return mode == 1 ? occupancy_rows_once<CK, false, WPE>() : occupancy_rows_once<CK, true, WPE>();
 }
 
 // Row-streamed partial-sum kernels for the 2D boxes of radius >= 2 (whose
@@ -156,7 +100,6 @@ void add_rows(std::vector<Variant>& out) {
     v.regcap = WPE > 0 ? 512 / WPE : 0;
     v.fn[1] = &launch_rows<CK, true, WPE>;
     v.fn_fast[1] = &launch_rows<CK, false, WPE>;
-    v.occ[1] = &occupancy_rows<CK, WPE>;
     out.push_back(v);
   }
 }
@@ -165,21 +108,6 @@ template <int CK, int CJ, int NW, bool EXACT>
 hipError_t launch_rows3(const LaunchArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t st) {
   hipLaunchKernelGGL((rows3_kernel<SID, T, CK, CJ, NW, EXACT>), grid, block, 0, st, to_args<T>(a));
   return hipGetLastError();
-}
-
-template <int CK, int CJ, int NW, bool EXACT>
-int occupancy_rows3_once() {
-  static const int n = [] {
-    int blocks = 0;
-    const void* k = reinterpret_cast<const void*>(&rows3_kernel<SID, T, CK, CJ, NW, EXACT>);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 64 * NW, 0) != hipSuccess) return 0;
-    return blocks;
-  }();
-  return n;
-}
-template <int CK, int CJ, int NW>
-int occupancy_rows3(int mode) {
-  return mode == 1 ? occupancy_rows3_once<CK, CJ, NW, false>() : occupancy_rows3_once<CK, CJ, NW, true>();
 }
 
 // Plane-streamed partial sums for the radius-1 3D boxes (taps grouped by
@@ -195,7 +123,6 @@ void add_rows3(std::vector<Variant>& out) {
     v.ck = CK; v.cj = CJ; v.nw = NW; v.btmax = 1;
     v.fn[1] = &launch_rows3<CK, CJ, NW, true>;
     v.fn_fast[1] = &launch_rows3<CK, CJ, NW, false>;
-    v.occ[1] = &occupancy_rows3<CK, CJ, NW>;
     out.push_back(v);
   }
 }
@@ -228,7 +155,6 @@ void add_sweep(std::vector<Variant>& out) {
         v.fn_share[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, false, true>;
         v.share_scratch[BT] = &share_scratch_once<BT, sh.ck, sh.cj, sh.nw>;
       }
-      v.occ[BT] = &occupancy_sweep<BT, sh.ck, sh.cj, sh.nw>;
       // intermediate-stage outputs: the adjoint's checkpointing forward pass (2D, exact)
       if constexpr (Def<SID>::dim == 2 && BT >= 2 && BT <= kMaxMidBT)
         v.fn_mid[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, true>;
@@ -261,7 +187,6 @@ void add_capped(std::vector<Variant>& out) {
       v.lds[BT] = sweep_lds_bytes<SID, T, sh.ck, sh.cj, sh.nw>(BT);
       v.fn[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, false, false, C>;
       v.fn_fast[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, false, false, false, C>;
-      v.occ[BT] = &occupancy_sweep<BT, sh.ck, sh.cj, sh.nw, C>;
       if constexpr (Def<SID>::dim == 2 && BT >= 2 && BT <= kMaxMidBT)
         v.fn_mid[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, true>;
     });
@@ -302,7 +227,6 @@ void AN5D_CAT(register_variants_, AN5D_SID, AN5D_F64)(std::vector<Variant>& out)
     pv.lds[1] = plane_lds_bytes<T, CK, CJ, NW, Def<SID>::rad>();
     pv.fn[1] = &launch_plane<CK, CJ, NW, true>;
     pv.fn_fast[1] = &launch_plane<CK, CJ, NW, false>;
-    pv.occ[1] = &occupancy_plane<CK, CJ, NW>;
     out.push_back(pv);
   }
   // register-capped twins of the sweep shapes, after the other variants so
