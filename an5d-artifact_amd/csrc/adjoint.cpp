@@ -88,6 +88,13 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
   int rc = resolve(p, &fc, &ap.fwd, &bt_pref, &sl_pref);
   if (rc) return rc;
   int bt = cfg && cfg->bt > 0 ? cfg->bt : ap.adj->btmax;
+  // a tuned choice that is shallower than the block (the one-step kernels) gives
+  // way to the stencil's sweep
+  if ((!cfg || cfg->variant < 0) && ap.fwd->btmax < bt && vs[0]->btmax >= bt) {
+    ap.fwd = vs[0];
+    bt_pref = bt;
+    sl_pref = 0;
+  }
   if (bt > ap.adj->btmax || bt > ap.fwd->btmax) {
     if (cfg && cfg->bt > 0) return fail(AN5D_E_UNSUPPORTED, "bt exceeds the adjoint or forward btmax");
     bt = ap.adj->btmax < ap.fwd->btmax ? ap.adj->btmax : ap.fwd->btmax;

@@ -36,13 +36,12 @@ int hip_fail(hipError_t e, const char* what) {
   void register_variants_##id##_0(std::vector<Variant>&);     \
   void register_variants_##id##_1(std::vector<Variant>&);
 AN5D_STENCILS(AN5D_DECL_REG)
-// cols_inst.hip
-void register_cols_17_0(std::vector<Variant>&);
-void register_cols_17_1(std::vector<Variant>&);
-void register_cols_18_0(std::vector<Variant>&);
-void register_cols_18_1(std::vector<Variant>&);
-void register_cols_19_0(std::vector<Variant>&);
-void register_cols_19_1(std::vector<Variant>&);
+// cols_inst.hip: the stencils the Makefile builds it for
+#define AN5D_COLS_IDS(X) X(5) X(6) X(7) X(17) X(18) X(19)
+#define AN5D_DECL_COLS(id)                            \
+  void register_cols_##id##_0(std::vector<Variant>&); \
+  void register_cols_##id##_1(std::vector<Variant>&);
+AN5D_COLS_IDS(AN5D_DECL_COLS)
 
 std::vector<Variant>& registry() {
   static std::vector<Variant> v = [] {
@@ -52,12 +51,10 @@ std::vector<Variant>& registry() {
   register_variants_##id##_1(out);
     AN5D_STENCILS(AN5D_CALL_REG)
     // after the others, so the indices of those stay put
-    register_cols_17_0(out);
-    register_cols_17_1(out);
-    register_cols_18_0(out);
-    register_cols_18_1(out);
-    register_cols_19_0(out);
-    register_cols_19_1(out);
+#define AN5D_CALL_COLS(id)    \
+  register_cols_##id##_0(out); \
+  register_cols_##id##_1(out);
+    AN5D_COLS_IDS(AN5D_CALL_COLS)
     return out;
   }();
   return v;
@@ -213,9 +210,22 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     return true;
   }
   if (v.kind == kCols) {
+    if (nk < v.ck) { err = "rows shorter than a lane's run"; return false; }
+    if (g.dim == 2) {
+      // lanes of ck cells over the segments, row-major
+      const long long ntk = cdiv(nk, v.ck);
+      if (sl <= 0) sl = default_sl(v, bt, g, ntk, 1);
+      if (sl > n0) sl = (int)n0;
+      const long long nseg = cdiv(n0, sl);
+      if (ntk * nseg >= (1LL << 30)) { err = "grid too large"; return false; }
+      a.ntk = (int)ntk; a.ntj = 1; a.nseg = (int)nseg; a.sl = sl;
+      a.SK = v.ck; a.SJ = 1;
+      lp.block = dim3(256);
+      lp.grid = dim3((unsigned)cdiv(ntk * nseg, 256));
+      return true;
+    }
     // lanes of ck cells over the plane, row-major, in blocks of 256 per segment
     const long long ntk = cdiv(nk, v.ck), nblk = cdiv(ntk * nj, 256);
-    if (nk < v.ck) { err = "rows shorter than a lane's run"; return false; }
     if (ntk * nj >= (1LL << 30)) { err = "grid too large"; return false; }
     if (sl <= 0) sl = default_sl(v, bt, g, nblk, 1);
     const long long nseg = cdiv(n0, sl);
@@ -622,7 +632,7 @@ int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout,
     if (share && v->fn_share[k] && v->share_scratch[k] && v->share_scratch[k]() == 0) return kLaunchShare;
     return rcfg.mode;
   };
-  if (v->kind == kCols) cols_coefs(p, cbytes, rcfg.mode);
+  if (v->kind == kCols && g.dim == 3) cols_coefs(p, cbytes, rcfg.mode);
   const void* dcoef = nullptr;
   rc = device_coefs(cbytes, &dcoef);
   if (rc) return rc;

@@ -142,7 +142,7 @@ double model_gstencil(const an5d_problem* p, const Variant& v, int bt, int sl, i
     ovi = (lp.args.nseg * (double)lp.args.sl + 2.0 * bt * g.r * lp.args.nseg) / n0;
     waves = (double)lp.args.ntk * lp.args.ntj * lp.args.nseg * (g.dim == 3 ? v.nw : 1);
   } else if (v.kind == kCols) {
-    waves = (double)lp.args.ntj * lp.args.nseg * 4;
+    waves = g.dim == 3 ? (double)lp.args.ntj * lp.args.nseg * 4 : (double)lp.args.ntk * lp.args.nseg / 64;
     ovi = (lp.args.sl + 0.5 * g.r) / lp.args.sl;
   } else if (v.kind == kPlane) {
     ovk = lp.args.ntk * 64.0 * v.ck / nk;

@@ -1,7 +1,7 @@
-// Instantiates and registers the column kernels of one 3D box x dtype
+// Instantiates and registers the column kernels of one box x dtype
 // (-DAN5D_SID=<stencil id> -DAN5D_F64=<0|1>).
 #include "cols.hpp"
-#include "engine.hpp"
+#include "cols2.hpp"
 #include "launch.hpp"
 
 namespace an5d {
@@ -11,8 +11,15 @@ using T = std::conditional_t<AN5D_F64, double, float>;
 constexpr int SID = AN5D_SID;
 
 template <int CK, bool EXACT>
+constexpr auto cols_fn() {
+  if constexpr (Def<SID>::dim == 3) return &cols_kernel<SID, T, CK, EXACT>;
+  else return &cols2_kernel<SID, T, CK, EXACT>;
+}
+
+template <int CK, bool EXACT>
 hipError_t launch_cols(const LaunchArgs& a, dim3 grid, dim3 block, size_t, hipStream_t st) {
-  hipLaunchKernelGGL((cols_kernel<SID, T, CK, EXACT>), grid, block, 0, st, to_args<T>(a));
+  constexpr auto kern = cols_fn<CK, EXACT>();
+  hipLaunchKernelGGL(kern, grid, block, 0, st, to_args<T>(a));
   return hipGetLastError();
 }
 

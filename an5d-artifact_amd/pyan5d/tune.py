@@ -1,6 +1,11 @@
 """Build the autotuner table for a set of workloads on the current GPU.
 
-    python -m pyan5d.tune [--set bench|all] [--out FILE] [--max-measured K]
+    python -m pyan5d.tune [--set bench|ladder|all] [--stencils A,B] [--out FILE] [--max-measured K]
+
+"ladder": every stencil, dtype and mode at sides of powers of two, so that a
+grid of any size has a row of about its own cell count (the library takes the
+nearest one within 8x; kernel and depth carry over, the segment length is
+chosen for the grid at hand).  "all" is both sets.
 
 For every (stencil, dtype, size, mode, run length) of the set, an5d_autotune
 ranks all (kernel shape, register cap, bt, sl) candidates with the analytic
@@ -46,21 +51,27 @@ BENCH = [
 ]
 
 
+LADDER_2D = [256, 512, 1024, 2048, 4096, 8192, 16384]
+LADDER_3D = [64, 128, 256, 512]
+
+
 def workloads(which):
-    out = list(BENCH)
-    if which == "all":
-        seen = {(s, np.dtype(d).name, tuple(n), m) for s, d, n, ms, _ in BENCH for m in ms}
+    out = [] if which == "ladder" else list(BENCH)
+    if which in ("ladder", "all"):
+        seen = {(s, np.dtype(d).name, tuple(n), m) for s, d, n, ms, _ in out for m in ms}
         for s in STENCILS_2D + STENCILS_3D:
-            n = [16384, 16384] if s in STENCILS_2D else [512, 512, 512]
-            for dt in (np.float32, np.float64):
-                if (s, np.dtype(dt).name, tuple(n), EXACT) not in seen:
-                    out.append((s, dt, n, (EXACT,), 1000))
+            for n in [[x] * 2 for x in LADDER_2D] if s in STENCILS_2D else [[x] * 3 for x in LADDER_3D]:
+                for dt in (np.float32, np.float64):
+                    modes = tuple(m for m in (EXACT, FAST) if (s, np.dtype(dt).name, tuple(n), m) not in seen)
+                    if modes:
+                        out.append((s, dt, n, modes, 100))
     return out
 
 
 def main(argv=None):
     ap = argparse.ArgumentParser(description=__doc__.splitlines()[0])
-    ap.add_argument("--set", choices=("bench", "all"), default="all")
+    ap.add_argument("--set", choices=("bench", "ladder", "all"), default="all")
+    ap.add_argument("--stencils", default="", help="only these, comma-separated (default: every one of the set)")
     ap.add_argument("--out", default=None, help="table file (default: the library's tuned.tsv)")
     ap.add_argument("--max-measured", type=int, default=1000)
     ap.add_argument("--fresh", action="store_true", help="start from an empty table")
@@ -69,7 +80,10 @@ def main(argv=None):
         tune_clear()
     elif args.out and os.path.exists(args.out):
         tune_load(args.out)
+    only = [s for s in args.stencils.split(",") if s]
     for name, dt, n, modes, steps in workloads(args.set):
+        if only and name not in only:
+            continue
         info(name)  # validates the name
         for mode in modes:
             t0 = time.perf_counter()

@@ -203,3 +203,23 @@ def test_adjoint_workspace_beyond_device_memory_is_rejected(torch_cuda):
     print("case adjoint workspace too large", flush=True)
     with pytest.raises(pyan5d.An5dError, match="exceeds the device"):
         pyan5d.AdjointWorkspace("j2d5pt", [16384, 16384], 20000, np.float32, bt=1)
+
+
+@pytest.mark.parametrize("n", [[700, 900], [2000, 1500]])
+def test_adjoint_block_deeper_than_the_tuned_forward_kernel(n):
+    """Where the tuned forward choice is a one-step kernel (the wide boxes), the
+    adjoint still runs its own block depth."""
+    name, T = "box2d2r", 7
+    u0, target, c, div = problem(name, n, np.float32, seed=2)
+    print(f"case adjoint depth {name} {n}", flush=True)
+    whole = pyan5d.adjoint_host(name, u0, target, n, T, coefs=c, divisor=div)
+    for bt in (1, 2, 3):
+        loss, g, gc, _, _ = pyan5d.adjoint_host(name, u0, target, n, T, coefs=c, divisor=div, bt=bt)
+        assert loss == whole[0]
+        assert np.max(np.abs(g - whole[1])) <= 2e-4 * np.max(np.abs(whole[1]))
+        if bt == 3:
+            assert same_bits(gc, whole[2])
+
+
+def same_bits(a, b):
+    return np.array_equal(a.view(np.uint64), b.view(np.uint64))

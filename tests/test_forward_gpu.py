@@ -384,3 +384,25 @@ def test_direct_kernel_fast_mode_with_subtracted_taps(name, dt):
     O.run(name, B, n, T)
     got, ref = A[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
     assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("name", ["box2d2r", "box2d3r", "box2d4r"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_box2d_run_kernel_ragged_grids(name, dt):
+    """The run kernel of the wide 2D boxes (kind 4): one row, one run per row,
+    rows that end inside a run, a last segment that overlaps its neighbour,
+    more lanes than runs; bit for bit the oracle, also over a divisor, and
+    within 1e-5 / 1e-12 of the field's largest value in FMA mode."""
+    v, = [v for v in pyan5d.variants(name, 0 if dt == np.float32 else 1) if v["kind"] == 4]
+    for n, sl, div in [([1, 4], 0, -1.0), ([7, 5], 3, 7.0), ([23, 131], 5, -1.0), ([64, 258], 0, 118.0),
+                       ([50, 70], 16, -1.0)]:
+        T = 3
+        print(f"case runs {name} {np.dtype(dt).name} n={n} sl={sl} divisor={div}", flush=True)
+        A = rand_grid(name, n, dt, seed=sum(n))
+        B, C = A.copy(), A.copy()
+        pyan5d.forward_host(name, A, n, T, variant=v["index"], sl=sl, divisor=div)
+        O.run(name, B, n, T, divisor=div)
+        assert same(A[T % 2], B[T % 2])
+        pyan5d.forward_host(name, C, n, T, variant=v["index"], sl=sl, divisor=div, mode=pyan5d.FAST)
+        got, ref = C[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
+        assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
