@@ -109,7 +109,7 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
   // multiple stays within the tuned depth, m=2 won)
   int m = bt_pref / bt;
   if (m < 1) m = 1;
-  while (m > 1 && (m * bt > ap.fwd->btmax || m * bt > kMaxMidBT)) m--;
+  while (m > 1 && (m * bt > ap.fwd->btmax || m * bt > kMaxMidBT || !ap.fwd->fn_mid[m * bt])) m--;
   int btf = m * bt;
   if (ap.fwd->kind == kDirect) btf = 1;
   ap.btf = btf;

@@ -36,12 +36,17 @@ int hip_fail(hipError_t e, const char* what) {
   void register_variants_##id##_0(std::vector<Variant>&);     \
   void register_variants_##id##_1(std::vector<Variant>&);
 AN5D_STENCILS(AN5D_DECL_REG)
-// cols_inst.hip: the stencils the Makefile builds it for
+// cols_inst.hip, tile2_inst.hip: the stencils the Makefile builds them for
 #define AN5D_COLS_IDS(X) X(5) X(6) X(7) X(17) X(18) X(19)
+#define AN5D_TILE_IDS(X) X(0) X(1) X(2) X(3) X(4) X(5) X(8) X(9) X(10) X(11)
 #define AN5D_DECL_COLS(id)                            \
   void register_cols_##id##_0(std::vector<Variant>&); \
   void register_cols_##id##_1(std::vector<Variant>&);
+#define AN5D_DECL_TILE(id)                             \
+  void register_tile2_##id##_0(std::vector<Variant>&); \
+  void register_tile2_##id##_1(std::vector<Variant>&);
 AN5D_COLS_IDS(AN5D_DECL_COLS)
+AN5D_TILE_IDS(AN5D_DECL_TILE)
 
 std::vector<Variant>& registry() {
   static std::vector<Variant> v = [] {
@@ -54,7 +59,11 @@ std::vector<Variant>& registry() {
 #define AN5D_CALL_COLS(id)    \
   register_cols_##id##_0(out); \
   register_cols_##id##_1(out);
+#define AN5D_CALL_TILE(id)     \
+  register_tile2_##id##_0(out); \
+  register_tile2_##id##_1(out);
     AN5D_COLS_IDS(AN5D_CALL_COLS)
+    AN5D_TILE_IDS(AN5D_CALL_TILE)
     return out;
   }();
   return v;
@@ -201,6 +210,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     lp.fn = mode == AN5D_FAST ? v.fn_fast[bt] : (mode == kLaunchShare ? v.fn_share[bt] : v.fn[bt]);
   if (!lp.fn) { err = "no kernel for bt=" + std::to_string(bt) + " in this variant"; return false; }
   lp.lds = (bt >= 1 && bt <= kMaxBT) ? v.lds[bt] : 0;
+  a.steps = bt;
   if (v.kind == kDirect) {
     const long long total = cdiv(nk, v.ck) * nj * n0;
     lp.block = dim3(256);
@@ -234,6 +244,20 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     lp.block = dim3(256);
     if (nblk * nseg >= (1LL << 31)) { err = "grid too large"; return false; }
     lp.grid = dim3((unsigned)(nblk * nseg));
+    return true;
+  }
+  if (v.kind == kTile) {
+    // tiles of nw*cj rows x 64*ck cells that give up bt*R cells on every side
+    // but the grid's own edges
+    const long long TH = (long long)v.nw * v.cj, TW = 64LL * v.ck, H = (long long)bt * R;
+    if (TH <= 2 * H || TW <= 2 * H) { err = "bt too deep for this variant's tile"; return false; }
+    const long long nti = g.D0 > TH ? cdiv(g.D0 - 2 * H, TH - 2 * H) : 1;
+    const long long ntk = g.D2 > TW ? cdiv(g.D2 - 2 * H, TW - 2 * H) : 1;
+    if (nti * ntk >= (1LL << 31)) { err = "grid too large"; return false; }
+    a.ntk = (int)ntk; a.ntj = 1; a.nseg = (int)nti; a.sl = (int)(TH - 2 * H);
+    a.SK = (int)(TW - 2 * H); a.SJ = (int)(TH - 2 * H);
+    lp.block = dim3(64 * v.nw);
+    lp.grid = dim3((unsigned)(nti * ntk));
     return true;
   }
   if (v.kind == kPlane) {

@@ -110,7 +110,7 @@ double ops_per_update(const StencilRT& s, const Variant& v, int mode, bool has_d
   if (!s.linear) ops = 45.0;
   else if (mode == AN5D_FAST) ops = s.ntaps;
   else ops = 2.0 * s.ntaps - 1 + (has_div ? 6.0 : 0.0);
-  if (v.kind == kSweep || v.kind == kRows) {
+  if (v.kind == kSweep || v.kind == kRows || v.kind == kTile) {
     // DPP halo per row and the middle-dim exchange, per cell
     ops += 2.0 * s.rad / v.ck;
     if (s.dim == 3) ops += 2.0 * s.rad * 2.0 / v.cj;
@@ -144,6 +144,10 @@ double model_gstencil(const an5d_problem* p, const Variant& v, int bt, int sl, i
   } else if (v.kind == kCols) {
     waves = g.dim == 3 ? (double)lp.args.ntj * lp.args.nseg * 4 : (double)lp.args.ntk * lp.args.nseg / 64;
     ovi = (lp.args.sl + 0.5 * g.r) / lp.args.sl;
+  } else if (v.kind == kTile) {
+    ovk = lp.args.ntk * 64.0 * v.ck / nk;
+    ovi = lp.args.nseg * (double)v.nw * v.cj / n0;
+    waves = (double)lp.args.ntk * lp.args.nseg * v.nw;
   } else if (v.kind == kPlane) {
     ovk = lp.args.ntk * 64.0 * v.ck / nk;
     ovj = lp.args.ntj * (double)v.nw * v.cj / nj;
@@ -215,7 +219,7 @@ extern "C" int an5d_autotune(const an5d_problem* p, void* dA, const an5d_layout*
     const Variant& v = *vs[vi];
     for (int bt = 1; bt <= v.btmax; bt++) {
       for (int sl : sls) {
-        if (v.kind == kDirect && sl != 0) continue;
+        if ((v.kind == kDirect || v.kind == kTile) && sl != 0) continue;
         if (sl > n0) continue;
         LaunchPlan lp;
         if (!plan_launch(v, bt, g, sl, lp, err, mode)) continue;

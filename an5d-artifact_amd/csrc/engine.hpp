@@ -36,7 +36,8 @@ inline hipError_t lds_opt_in(const void* kernel, size_t lds, std::atomic<int>* d
 // kCols: one step per launch, a column (3D) or run (2D) of cells per lane, for
 // the boxes of radius >= 2; in 3D its coefficient table has an order of its own
 // (cols_coefs)
-enum KernelKind { kSweep = 0, kDirect = 1, kPlane = 2, kRows = 3, kCols = 4 };
+// kTile: several steps per launch on a 2D tile held in registers
+enum KernelKind { kSweep = 0, kDirect = 1, kPlane = 2, kRows = 3, kCols = 4, kTile = 5 };
 enum DType { kF32 = 0, kF64 = 1 };
 
 // dtype-erased SweepArgs<T>
@@ -54,6 +55,7 @@ struct LaunchArgs {
   long long mid_stride;  // elements between consecutive intermediate outputs
   unsigned mid_mask;     // bit S: store stage S; 0: none
   int nt_store;          // 1: non-temporal stores for shallow blocks
+  int steps;             // steps of this launch (kernels that take them at run time)
 };
 
 using LaunchFn = hipError_t (*)(const LaunchArgs&, dim3 grid, dim3 block, size_t lds,

@@ -22,6 +22,7 @@ SweepArgs<U> to_args(const LaunchArgs& a) {
   s.mid_stride = a.mid_stride;
   s.mid_mask = a.mid_mask;
   s.nt_store = a.nt_store;
+  s.steps = a.steps;
   return s;
 }
 

@@ -54,6 +54,7 @@ struct SweepArgs {
   long long mid_stride;
   unsigned mid_mask;
   int nt_store;  // 1: non-temporal stores (grid larger than the last-level cache)
+  int steps;     // steps of the launch, where the kernel takes them at run time
 };
 
 // ---- cross-lane moves ------------------------------------------------------

@@ -71,6 +71,7 @@ FIELDS = {
     "rows3_kernel": ["ck", "cj", "nw", "exact"],
     "cols_kernel": ["ck", "exact"],
     "cols2_kernel": ["ck", "exact"],
+    "tile2_kernel": ["ck", "cj", "nw", "exact"],
 }
 
 

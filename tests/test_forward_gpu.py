@@ -406,3 +406,30 @@ def test_box2d_run_kernel_ragged_grids(name, dt):
         pyan5d.forward_host(name, C, n, T, variant=v["index"], sl=sl, divisor=div, mode=pyan5d.FAST)
         got, ref = C[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
         assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
+
+
+TILE_NAMES = ["star2d1r", "star2d2r", "star2d3r", "star2d4r", "box2d1r", "box2d2r", "j2d5pt", "j2d9pt",
+              "j2d9pt-gol", "gradient2d"]
+
+
+@pytest.mark.parametrize("name", TILE_NAMES)
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_register_tiles_at_their_edges(name, dt):
+    """The register-tile kernels (kind 5): a grid of one cell, of exactly one
+    tile, one cell more in either direction (two tiles, the second owning
+    little), several tiles; the deepest block and one that is not; bit for bit
+    the oracle."""
+    r = O.info(name)["rad"]
+    for v in pyan5d.variants(name, 0 if dt == np.float32 else 1):
+        if v["kind"] != 5:
+            continue
+        th, tw = v["nw"] * v["cj"] - 2 * r, 64 * v["ck"] - 2 * r  # interior of a grid that is one tile
+        for bt in sorted({1, max(1, v["btmax"] // 2), v["btmax"]}):
+            for n in ([1, 1], [th, tw], [th + 1, tw], [th, tw + 1], [2 * th + 5, tw + 70]):
+                T = bt + max(1, bt // 2)
+                print(f"case tiles {name} {np.dtype(dt).name} variant {v['index']} bt={bt} n={n}", flush=True)
+                A = rand_grid(name, n, dt, seed=sum(n) + bt)
+                B = A.copy()
+                pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt)
+                O.run(name, B, n, T)
+                assert same(A[T % 2], B[T % 2])
