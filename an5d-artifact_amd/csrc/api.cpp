@@ -15,6 +15,7 @@
 #include "../../include/an5d.h"
 #include "engine.hpp"
 #include "internal.hpp"
+#include "staging.hpp"
 #include "stencil_defs.hpp"
 
 namespace an5d {
@@ -122,15 +123,6 @@ an5d_layout reference_layout(const Geom& g) {
   L.s1 = g.D2;
   L.s0 = g.D1 * g.D2;
   L.buf_stride = g.area;
-  return L;
-}
-
-an5d_layout padded_layout(const Geom& g) {
-  an5d_layout L;
-  const long long pitch = (g.D2 + 63) / 64 * 64;  // 256-byte (FP32) rows
-  L.s1 = pitch;
-  L.s0 = g.D1 * pitch;
-  L.buf_stride = g.D0 * L.s0;
   return L;
 }
 
@@ -405,7 +397,8 @@ struct DeviceCache {
   std::mutex mu;
   std::map<std::pair<int, std::string>, void*> coefs;  // (device, bytes) -> device copy
   std::map<int, std::pair<void*, size_t>> grids;       // device -> staging grid buffer
-  std::map<int, std::mutex> grid_users;                // device -> holder of its staging grid
+  std::map<int, Staging> stagings;                     // device -> pinned ring of its transfers
+  std::map<int, std::mutex> grid_users;                // device -> holder of its staging grid and ring
 };
 static DeviceCache& cache() {
   static DeviceCache* c = new DeviceCache();
@@ -434,7 +427,7 @@ int device_coefs(const std::vector<unsigned char>& bytes, const void** out) {
   return AN5D_OK;
 }
 
-int device_grid(size_t bytes, void** out, std::unique_lock<std::mutex>& hold) {
+int device_grid(size_t bytes, void** out, Staging** ring, std::unique_lock<std::mutex>& hold) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
@@ -457,7 +450,8 @@ int device_grid(size_t bytes, void** out, std::unique_lock<std::mutex>& hold) {
     slot = {d, bytes};
   }
   *out = slot.first;
-  return AN5D_OK;
+  *ring = &c.stagings[dev];  // map nodes stay put
+  return staging_init(**ring);
 }
 
 // ---- variant / bt resolution ---------------------------------------------------
@@ -626,7 +620,7 @@ extern "C" int an5d_variant_get_info(int stencil, int dtype, int variant, an5d_v
 namespace an5d {
 
 int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout,
-                 const an5d_config* cfg, int steps_only, int c0_first, hipStream_t st) {
+                 const an5d_config* cfg, int steps_only, int c0_first, hipStream_t st, int* launches) {
   Geom g;
   std::string err;
   if (!make_geom(p, g, err)) return fail(AN5D_E_INVALID, err);
@@ -670,6 +664,7 @@ int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout,
     steps.resize(n);
     an5d_schedule(p->timesteps, v->kind == kDirect ? 1 : bt, steps.data(), n);
   }
+  if (launches) *launches = (int)steps.size();
   int c0 = c0_first;
   // one plan per distinct step count (a schedule has at most three)
   LaunchPlan plans[kMaxBT + 1];
@@ -729,32 +724,36 @@ extern "C" int an5d_forward_host(const an5d_problem* p, void* A, const an5d_conf
   if (p->timesteps < 0) return fail(AN5D_E_INVALID, "timesteps must be >= 0");
   if (p->timesteps == 0) return AN5D_OK;
   const size_t esz = p->dtype == AN5D_FLOAT64 ? 8 : 4;
-  an5d_layout L = padded_layout(g);
+  const size_t gb = (size_t)g.area * esz;
   void* dA = nullptr;
-  std::unique_lock<std::mutex> hold;  // the staging grid is ours until we return
-  int rc = device_grid((size_t)2 * L.buf_stride * esz, &dA, hold);
+  Staging* ring = nullptr;
+  std::unique_lock<std::mutex> hold;  // the staging grid and ring are ours until we return
+  int rc = device_grid(2 * gb, &dA, &ring, hold);
   if (rc) return rc;
-  const size_t rows = (size_t)g.D0 * g.D1;
-  hipError_t e;
-  for (int b = 0; b < 2; b++) {
-    e = hipMemcpy2D(static_cast<char*>(dA) + (size_t)b * L.buf_stride * esz, L.s1 * esz,
-                    static_cast<char*>(A) + (size_t)b * g.area * esz, g.D2 * esz, g.D2 * esz, rows,
-                    hipMemcpyHostToDevice);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpy2D H2D");
-  }
-  e = hipDeviceSynchronize();
-  if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
+  char* h0 = static_cast<char*>(A);
+  char* h1 = h0 + gb;
+  char* d0 = static_cast<char*>(dA);
+  char* d1 = d0 + gb;
+  // The first launch writes the whole interior of buffer 1: of that buffer only
+  // the halo is read, so only the halo goes up.
+  rc = staging_upload(*ring, d0, h0, gb);
+  if (rc == AN5D_OK) rc = staging_upload_halo(*ring, d1, h1, g, esz);
+  hipError_t e = hipStreamSynchronize(ring->st);
+  if (rc) return rc;
+  if (e != hipSuccess) return hip_fail(e, "H2D copies");
+  int launches = 0;
   const double t0 = sb_time_ms();
-  rc = run_schedule(p, dA, &L, cfg, 0, 0, nullptr);
-  if (rc) return rc;
-  e = hipDeviceSynchronize();
+  rc = run_schedule(p, dA, nullptr, cfg, 0, 0, ring->st, &launches);
+  e = hipStreamSynchronize(ring->st);
   const double t1 = sb_time_ms();
+  if (rc) return rc;
   if (e != hipSuccess) return hip_fail(e, "kernel execution");
-  for (int b = 0; b < 2; b++) {
-    e = hipMemcpy2D(static_cast<char*>(A) + (size_t)b * g.area * esz, g.D2 * esz,
-                    static_cast<char*>(dA) + (size_t)b * L.buf_stride * esz, L.s1 * esz, g.D2 * esz,
-                    rows, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpy2D D2H");
+  // a single launch leaves buffer 0 as it came
+  if (launches > 1) rc = staging_download(*ring, h0, d0, gb);
+  if (rc == AN5D_OK) rc = staging_download(*ring, h1, d1, gb);
+  if (rc) {
+    (void)hipStreamSynchronize(ring->st);
+    return rc;
   }
   if (ms) *ms = t1 - t0;
   return AN5D_OK;
@@ -789,12 +788,23 @@ extern "C" int an5d_kernel_stencil(int stencil, int dtype, void* A1, int compsiz
 
 extern "C" int an5d_release(void) {
   DeviceCache& c = cache();
+  // host calls under way keep their grid and ring until they return
+  std::vector<std::unique_lock<std::mutex>> users;
+  {
+    std::vector<std::mutex*> all;
+    {
+      std::lock_guard<std::mutex> lk(c.mu);
+      for (auto& kv : c.grid_users) all.push_back(&kv.second);
+    }
+    for (std::mutex* m : all) users.emplace_back(*m);
+  }
   std::lock_guard<std::mutex> lk(c.mu);
   for (auto& kv : c.coefs) (void)hipFree(kv.second);
   c.coefs.clear();
   for (auto& kv : c.grids)
     if (kv.second.first) (void)hipFree(kv.second.first);
   c.grids.clear();
+  for (auto& kv : c.stagings) staging_free(kv.second);
   return AN5D_OK;
 }
 

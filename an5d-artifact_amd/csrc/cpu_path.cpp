@@ -22,7 +22,47 @@
 
 namespace an5d {
 int fail(int code, const std::string& msg);  // api.cpp: sets an5d_last_error()
+
+// ---- helpers of the staged transfers (staging.hpp) ---------------------------
+// Shares below 64 KB cost more to hand out than to copy.
+void parallel_copy(void* dst, const void* src, size_t bytes) {
+  const long long parts = (long long)(bytes / (64 << 10));
+  if (parts < 2) {
+    memcpy(dst, src, bytes);
+    return;
+  }
+#pragma omp parallel
+  {
+    const size_t nt = omp_get_num_threads(), t = omp_get_thread_num();
+    const size_t share = (bytes / nt + 63) / 64 * 64;
+    const size_t a = t * share < bytes ? t * share : bytes;
+    const size_t b = t + 1 == nt || a + share > bytes ? bytes : a + share;
+    memcpy(static_cast<char*>(dst) + a, static_cast<const char*>(src) + a, b - a);
+  }
 }
+
+void pack_side_halo(char* dst, const char* grid, int dim, long long r, long long D1, long long D2, size_t esz,
+                         long long i0, long long i1) {
+  const size_t row = (size_t)D2 * esz, end = (size_t)r * esz, plane = (size_t)D1 * row;
+  const size_t side = dim == 3 ? 2 * r * row + (size_t)(D1 - 2 * r) * 2 * end : 2 * end;
+#pragma omp parallel for schedule(static) if ((i1 - i0) * side > (64 << 10))
+  for (long long i = i0; i < i1; i++) {
+    char* o = dst + (size_t)(i - i0) * side;
+    const char* p = grid + (size_t)i * plane;
+    if (dim == 3) {
+      memcpy(o, p, r * row);
+      memcpy(o + r * row, p + plane - r * row, r * row);
+      o += 2 * r * row;
+      p += r * row;
+    }
+    const long long rows = dim == 3 ? D1 - 2 * r : 1;
+    for (long long j = 0; j < rows; j++, o += 2 * end, p += row) {
+      memcpy(o, p, end);
+      memcpy(o + end, p + row - end, end);
+    }
+  }
+}
+}  // namespace an5d
 
 namespace {
 

@@ -40,7 +40,6 @@ const StencilRT& stencil_rt(int id);
 std::vector<const Variant*> variants_of(int stencil, int dtype);
 bool make_geom(const an5d_problem* p, Geom& g, std::string& err);
 an5d_layout reference_layout(const Geom& g);
-an5d_layout padded_layout(const Geom& g);
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,
             int* slout);
 // plan_launch's mode: AN5D_EXACT, AN5D_FAST, or kLaunchShare (exact, the
@@ -53,11 +52,14 @@ bool build_coefs(const an5d_problem* p, std::vector<unsigned char>& bytes, int& 
                  double& gscale, std::string& err, int mode = 0);
 void cols_coefs(const an5d_problem* p, std::vector<unsigned char>& bytes, int mode);
 int device_coefs(const std::vector<unsigned char>& bytes, const void** out);
-// The current device's staging grid of at least `bytes`; `hold` keeps other
-// host calls on that device from using or regrowing it until released.
-int device_grid(size_t bytes, void** out, std::unique_lock<std::mutex>& hold);
-int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout,
-                 const an5d_config* cfg, int steps_only, int c0_first, hipStream_t st);
+// The current device's staging grid of at least `bytes` and its ring of pinned
+// buffers; `hold` keeps other host calls on that device from using or
+// regrowing them until released.
+struct Staging;
+int device_grid(size_t bytes, void** out, Staging** ring, std::unique_lock<std::mutex>& hold);
+// *launches (optional): the kernel launches the schedule has
+int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout, const an5d_config* cfg,
+                 int steps_only, int c0_first, hipStream_t st, int* launches = nullptr);
 double sb_time_ms();
 int device_cus();  // compute units of the current device (0 if unknown)
 

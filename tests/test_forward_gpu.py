@@ -433,3 +433,23 @@ def test_register_tiles_at_their_edges(name, dt):
                 pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt)
                 O.run(name, B, n, T)
                 assert same(A[T % 2], B[T % 2])
+
+
+@pytest.mark.parametrize("name,n", [("star2d2r", [1500, 3000]), ("star2d1r", [3, 5]), ("star3d2r", [30, 41, 53]),
+                                    ("box3d1r", [1, 2, 3])])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_host_arrays_with_two_halos(name, n, dt):
+    """Host arrays whose buffers hold different halos: every step reads the
+    halo of its own input buffer and writes none (bt = 1, so the C loop does
+    the same); both buffers come back, also after a single launch; arrays
+    beyond the pinned ring and of a few cells."""
+    r = O.info(name)["rad"]
+    rng = np.random.default_rng(6)
+    A0 = rng.random([2] + [x + 2 * r for x in n]).astype(dt)
+    for T in (1, 2, 3):
+        print(f"case host halos {name} {np.dtype(dt).name} {n} T={T}", flush=True)
+        A, B = A0.copy(), A0.copy()
+        pyan5d.forward_host(name, A, n, T, bt=1)
+        O.run(name, B, n, T)
+        # the schedule may end with fewer launches than steps only for bt > 1
+        assert same(A, B)
