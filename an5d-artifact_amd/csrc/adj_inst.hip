@@ -1,5 +1,6 @@
 // Instantiates and registers the adjoint kernels of one 2D stencil x dtype
 // (-DAN5D_SID=<stencil id> -DAN5D_F64=<0|1>).
+#include "adj_tile.hpp"
 #include "adjoint.hpp"
 #include "engine.hpp"
 
@@ -24,8 +25,7 @@ constexpr int adj_btmax() {
   return 1;
 }
 
-template <int BT>
-hipError_t launch_adj(const AdjLaunch& l, dim3 grid, dim3 block, hipStream_t st) {
+AdjArgs<T> to_adj_args(const AdjLaunch& l) {
   AdjArgs<T> a;
   a.U = static_cast<const T*>(l.U);
   a.Lin = static_cast<const T*>(l.Lin);
@@ -36,7 +36,12 @@ hipError_t launch_adj(const AdjLaunch& l, dim3 grid, dim3 block, hipStream_t st)
   a.gslot = l.gslot;
   a.D0 = l.D0; a.D2 = l.D2; a.s0 = l.s0;
   a.ntk = l.ntk; a.nseg = l.nseg; a.sl = l.sl; a.SK = l.SK;
-  hipLaunchKernelGGL((adjoint_kernel<SID, T, BT, adj_ck(), 4>), grid, block, 0, st, a);
+  return a;
+}
+
+template <int BT>
+hipError_t launch_adj(const AdjLaunch& l, dim3 grid, dim3 block, hipStream_t st) {
+  hipLaunchKernelGGL((adjoint_kernel<SID, T, BT, adj_ck(), 4>), grid, block, 0, st, to_adj_args(l));
   return hipGetLastError();
 }
 
@@ -57,6 +62,49 @@ int occupancy(int bt) {
   });
   return n;
 }
+
+// Register-tile shapes (adj_tile.hpp), FP64 stencils of up to 25 taps: 16 waves
+// of few cells for the smallest grids, 8 waves (whose 256 registers hold the
+// block's states, and less halo) above.  Left out: 16 waves for the box of
+// radius 2 (spills: 3199 us against 769 on 8 waves for 60 steps of 256^2); at
+// radius 3-4 the edge rows of a larger tile exceed LDS.
+template <int I>
+constexpr bool adj_tiled() {
+  if (!AN5D_F64 || !D::linear || D::ntaps > 25) return false;
+  return I == 0 ? D::ntaps <= 9 || D::rad >= 3 : D::rad <= 2;
+}
+template <int I> constexpr int tile_ck() { return D::rad >= 3 ? 4 : (I == 0 && D::rad == 1 ? 1 : 2); }
+template <int I> constexpr int tile_cj() { return I == 0 ? 2 : 4; }
+template <int I> constexpr int tile_nw() { return I == 1 || D::rad >= 3 ? 8 : 16; }
+
+template <int BT, int I>
+hipError_t launch_adj_tile(const AdjLaunch& l, dim3 grid, dim3 block, hipStream_t st) {
+  constexpr int CK = tile_ck<I>(), CJ = tile_cj<I>(), NW = tile_nw<I>();
+  constexpr size_t lds = adj_tile_lds_bytes<SID, T, CK, CJ, NW>();
+  constexpr auto kern = &adjoint_tile_kernel<SID, T, BT, CK, CJ, NW>;
+  static_assert(lds <= 160 * 1024, "edge rows exceed LDS");
+  if (lds > 65536) {
+    static std::atomic<int> done[kMaxDevices];
+    const hipError_t e = lds_opt_in(reinterpret_cast<const void*>(kern), lds, done);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(kern, grid, block, lds, st, to_adj_args(l));
+  return hipGetLastError();
+}
+
+template <int I>
+void add_tile(AdjVariant& v) {
+  if constexpr (adj_tiled<I>()) {
+    v.tile[I].ck = tile_ck<I>();
+    v.tile[I].cj = tile_cj<I>();
+    v.tile[I].nw = tile_nw<I>();
+    static_for<1, adj_btmax() + 1>([&](auto bc) {
+      constexpr int BT = decltype(bc)::value;
+      v.tile[I].fn[BT] = &launch_adj_tile<BT, I>;
+    });
+  }
+}
+
 hipError_t launch_seed(const void* uT, const void* target, void* lam, double* lslot, int D0, int D2,
                        long long s0, long long stgt, int R, hipStream_t st) {
   hipLaunchKernelGGL((adjoint_seed_kernel<T>), dim3(kSeedBlocks), dim3(256), 0, st, static_cast<const T*>(uT),
@@ -64,13 +112,14 @@ hipError_t launch_seed(const void* uT, const void* target, void* lam, double* ls
   return hipGetLastError();
 }
 
-hipError_t launch_halo(const void* src, void* dst, int D0, int D2, long long s0, int R, hipStream_t st) {
-  const long long cells = 2LL * R * D2 + 2LL * R * (D0 - 2 * R);
+hipError_t launch_halo(const void* src, void* dst, long long stride, int ndst, int D0, int D2, long long s0, int R,
+                       hipStream_t st) {
+  const long long cells = (2LL * R * D2 + 2LL * R * (D0 - 2 * R)) * ndst;
   long long blocks = (cells + 255) / 256;
   if (blocks > 1024) blocks = 1024;
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL((halo_copy_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, static_cast<const T*>(src),
-                     static_cast<T*>(dst), D0, D2, s0, R);
+                     static_cast<T*>(dst), stride, ndst, D0, D2, s0, R);
   return hipGetLastError();
 }
 
@@ -93,6 +142,8 @@ void AN5D_CAT(register_adjoint_, AN5D_SID, AN5D_F64)(std::vector<AdjVariant>& ou
     constexpr int BT = decltype(bc)::value;
     v.fn[BT] = &launch_adj<BT>;
   });
+  add_tile<0>(v);
+  add_tile<1>(v);
   out.push_back(v);
 }
 

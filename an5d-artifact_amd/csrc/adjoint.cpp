@@ -1,5 +1,6 @@
 // Adjoint entry points: checkpointed forward, seed, reverse block sweep.
 // No counterpart in the reference (it computes no gradients).
+#include <math.h>
 #include <string.h>
 
 #include <mutex>
@@ -63,11 +64,43 @@ struct AdjPlan {
   // seed kernel's per-wave loss slots (kSeedBlocks * 4 doubles)
   long long nslots = 0;
   int ng = 0;
+  bool rich = false;  // short streams and register tiles allowed
   size_t gslot_off = 0, lslot_off = 0;
 };
 
-static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, dim3& block,
-                           bool sizing = false);
+static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, dim3& block, AdjFn& fn,
+                           long long* slots = nullptr);
+
+// an5d_adjoint_device_noalloc's device array, and the part of it that holds
+// the coefficients (>= (81 taps + 2) * 8 bytes)
+constexpr size_t kNoAllocScratchBytes = 64ull << 20;
+constexpr size_t kNoAllocCoefBytes = 1024;
+static_assert(kNoAllocScratchBytes % 256 == 0, "scratch is carved in 256-byte units");
+
+// Shortest streamed segment.  Short segments and register tiles (FP64 only, see
+// adj_launch_plan) need a gradient slot each; a problem that would outgrow the
+// fixed scratch array by them alone keeps to the longer streams.
+constexpr long long kMinSl = 4, kMinSlLean = 16;
+
+// Gradient slots (the most any launch may use) and what follows them.
+static int plan_slots(AdjPlan& ap) {
+  ap.nslots = 0;
+  int seen = 0;
+  for (int k : ap.blocks) {
+    if (k == seen) continue;  // all but the last are alike
+    seen = k;
+    AdjLaunch l{};
+    dim3 grid, block;
+    AdjFn fn;
+    long long n = 0;
+    const int rc = adj_launch_plan(ap, k, l, grid, block, fn, &n);
+    if (rc) return rc;
+    if (n > ap.nslots) ap.nslots = n;
+  }
+  ap.lslot_off = ap.gslot_off + ((size_t)ap.nslots * ap.ng * sizeof(double) + 255) / 256 * 256;
+  ap.ws_bytes = ap.lslot_off + (size_t)kSeedBlocks * 4 * sizeof(double);
+  return AN5D_OK;
+}
 
 // The forward pass runs at its own temporal block btf (the largest multiple
 // of bt not above the tuned forward depth) and stores the state at every multiple of
@@ -125,21 +158,17 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
   const size_t esz = p->dtype == AN5D_FLOAT64 ? 8 : 4;
   ap.pitch = (ap.g.D2 + 2 * kPad + 63) / 64 * 64;
   ap.grid_bytes = ((size_t)(ap.g.D0 + 2 * kRowPad) * ap.pitch * esz + 255) / 256 * 256;
-  // gradient slots: the most wave tiles any adjoint launch uses
   ap.ng = stencil_rt(p->stencil).linear ? stencil_rt(p->stencil).ntaps : 2;
-  ap.nslots = 0;
-  for (int k : ap.blocks) {
-    AdjLaunch l{};
-    dim3 grid, block;
-    rc = adj_launch_plan(ap, k, l, grid, block, true);
-    if (rc) return rc;
-    const long long nt = (long long)l.ntk * l.nseg;
-    if (nt > ap.nslots) ap.nslots = nt;
-  }
   ap.gslot_off = ap.grid_bytes * (ap.blocks.size() + 1 + 2);
-  ap.lslot_off = ap.gslot_off + ((size_t)ap.nslots * ap.ng * sizeof(double) + 255) / 256 * 256;
-  ap.ws_bytes = ap.lslot_off + (size_t)kSeedBlocks * 4 * sizeof(double);
-  return AN5D_OK;
+  ap.rich = p->dtype == AN5D_FLOAT64;
+  rc = plan_slots(ap);
+  if (rc == AN5D_OK && ap.rich && ap.ws_bytes + kNoAllocCoefBytes > kNoAllocScratchBytes) {
+    AdjPlan lean = ap;
+    lean.rich = false;
+    rc = plan_slots(lean);
+    if (rc == AN5D_OK && lean.ws_bytes + kNoAllocCoefBytes <= kNoAllocScratchBytes) ap = lean;
+  }
+  return rc;
 }
 
 // Zeroes n doubles (a fill kernel rather than a memset node, so the call
@@ -178,42 +207,37 @@ __global__ __launch_bounds__(256) void adj_finish_kernel(const double* __restric
   }
 }
 
-// Segments along dim 0: by default as many as fill the GPU's resident wave
-// slots in one round (a second, partly filled round would leave most SIMDs
-// idle), at least kMinSl planes each.  `sizing` gives the most segments any
-// launch can use (the gradient-slot count) without touching the device.
-constexpr long long kMinSl = 16;
-static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, dim3& block,
-                           bool sizing) {
+// The launch of a k-step reverse block: the streamed kernel, or (FP64) a
+// register tile where the grid is too small to fill the chip with streams.
+//
+// FP32 lanes sum products in FP32 over a loop body before FP64 takes over, and
+// the bodies start at the segment's first plane: another segment length, or a
+// tile, regroups them and moves the coefficient gradient by 1e-8 (sums that
+// cancel).  FP32 therefore keeps its segments: as many as fill the resident
+// wave slots in one round, 16 planes at least.
+//
+// FP64: both kernels run the same stages on every cell; the model counts a
+// wave's cells per lane times the waves that share a SIMD on the busiest CU
+// (for a stream at least 2, for a tile 1.5: fewer leave latency exposed).  A
+// stream runs its sl planes, its warm-up and what fills whole ring lengths; a
+// tile runs its rows once, but extends and exchanges them anew at every step,
+// which costs kTileCost stream cells per cell (fitted, by radius and shape).
+// Forward + adjoint of 60 steps, streamed / small tile / large tile, us:
+//   j2d5pt      256^2 352/208/224  1024^2 557/584/425  2048^2 1417/1904/1338
+//   j2d9pt      256^2 569/546/465  1024^2 874/1050/916  2048^2 1806/3155/2654
+//   j2d9pt-gol  256^2 436/305/293  1024^2 715/943/595  2048^2 1436/2812/1706
+//   star2d4r    256^2 1423/1040    1024^2 1717/2369
+//   box2d2r     512^2 1187/-/784   1024^2 2199/-/1476   2048^2 4327/-/5334
+// With `slots` the call also counts the gradient slots any choice may need.
+static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, dim3& block, AdjFn& fn,
+                           long long* slots) {
   const int R = ap.g.r, W = ap.adj->reach;
-  const long long ck = ap.adj->ck;
+  const long long ck = ap.adj->ck, nw = ap.adj->nw;
   const long long HA = ((2LL * k - 2) * R + W + ck - 1) / ck * ck;  // whole lanes (adj_halo)
   const long long SK = 64LL * ap.adj->ck - 2 * HA;
   if (SK <= 0) return fail(AN5D_E_UNSUPPORTED, "adjoint block too deep for the tile");
   const long long nk = ap.g.D2 - 2 * R, n0 = ap.g.D0 - 2 * R;
   const long long ntk = cdiv(nk, SK);
-  long long sl = ap.sl;
-  if (sl <= 0) {
-    long long slots = 0;
-    if (!sizing) {
-      const int occ = ap.adj->occupancy ? ap.adj->occupancy(k) : 0;
-      slots = (long long)occ * device_cus() * ap.adj->nw;
-    }
-    if (sizing) {
-      sl = kMinSl;
-    } else if (slots > 0) {
-      const long long nseg = slots / ntk > 1 ? slots / ntk : 1;
-      sl = cdiv(n0, nseg);
-    } else {
-      sl = cdiv(n0, cdiv(4096, ntk));
-    }
-    if (sl < kMinSl) sl = kMinSl;
-  }
-  if (sl > n0) sl = n0;
-  const long long nseg = cdiv(n0, sl);
-  l.D0 = (int)ap.g.D0;
-  l.D2 = (int)ap.g.D2;
-  l.s0 = ap.pitch;
   // planes the kernel reads (see adjoint_kernel): checkpoint planes from
   // i0-HU on, lambda planes from i0-HU-DLT on (HU = 2(k-1)R+W,
   // DLT = W+(k-2)R), through i0+sle+DLT+k*R-1 plus the unrolled tail and the
@@ -225,12 +249,66 @@ static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, d
   const long long hi = (ap.g.D0 - R) + (DLT > 0 ? DLT : 0) + (long long)k * R + 2 * ring;
   if (lo < -kRowPad || hi >= ap.g.D0 + kRowPad || 64LL * ap.adj->ck > kPad)
     return fail(AN5D_E_UNSUPPORTED, "adjoint block reaches beyond the workspace padding");
+  const double cus = device_cus() > 0 ? device_cus() : 256;
+  const long long minsl = ap.rich ? kMinSl : kMinSlLean;
+  if (slots) *slots = ntk * cdiv(n0, ap.sl > 0 ? (ap.sl < n0 ? ap.sl : n0) : (minsl < n0 ? minsl : n0));
+  // streams
+  long long sl = ap.sl < n0 ? ap.sl : n0;
+  double t_best = 1e300;
+  if (ap.sl <= 0 && !ap.rich) {
+    const int occ = !slots && ap.adj->occupancy ? ap.adj->occupancy(k) : 0;
+    const long long resident = (long long)occ * device_cus() * nw;
+    const long long nseg = resident > 0 ? (resident / ntk > 1 ? resident / ntk : 1) : cdiv(4096, ntk);
+    sl = cdiv(n0, nseg);
+    if (sl < kMinSlLean) sl = kMinSlLean;
+    if (sl > n0) sl = n0;
+  } else if (ap.sl <= 0) {
+    for (long long nseg = 1; nseg <= n0; nseg++) {
+      const long long s = cdiv(n0, nseg);
+      if (s < minsl && nseg > 1) break;
+      const double share = ceil((double)cdiv(ntk * nseg, nw) / cus) * nw / 4;
+      const double planes = (double)cdiv(s + HU + DLT + k * R, ring - 1) * (ring - 1);
+      const double t = planes * ck * (share > 2.0 ? share : 2.0);
+      if (t < t_best) {
+        t_best = t;
+        sl = s;
+      }
+      if (share > 12) break;
+    }
+  }
+  l.D0 = (int)ap.g.D0;
+  l.D2 = (int)ap.g.D2;
+  l.s0 = ap.pitch;
   l.ntk = (int)ntk;
-  l.nseg = (int)nseg;
+  l.nseg = (int)cdiv(n0, sl);
   l.sl = (int)sl;
   l.SK = (int)SK;
-  block = dim3(64 * ap.adj->nw);
-  grid = dim3((unsigned)cdiv(ntk * nseg, ap.adj->nw));
+  block = dim3(64 * (unsigned)nw);
+  grid = dim3((unsigned)cdiv(ntk * l.nseg, nw));
+  fn = ap.adj->fn[k];
+  if (ap.sl > 0 || !ap.rich) return AN5D_OK;
+  constexpr double kTileCost[2][kAdjTiles] = {{4.0, 2.6}, {4.6, 3.8}};
+  // tiles (the padding rows and cells around the grid cover the last ones)
+  for (int i = 0; i < kAdjTiles; i++) {
+    const AdjTile& t = ap.adj->tile[i];
+    if (t.ck == 0 || !t.fn[k]) continue;
+    const long long TH = (long long)t.nw * t.cj, TW = 64LL * t.ck, H = (long long)k * R;
+    if (TH <= 2 * H || TW <= 2 * H || TH > kRowPad || TW > kPad) continue;
+    const long long nti = ap.g.D0 > TH ? cdiv(ap.g.D0 - 2 * H, TH - 2 * H) : 1;
+    const long long ntj = ap.g.D2 > TW ? cdiv(ap.g.D2 - 2 * H, TW - 2 * H) : 1;
+    if (slots && nti * ntj > *slots) *slots = nti * ntj;
+    const double share = ceil((double)(nti * ntj) / cus) * t.nw / 4;
+    const double time = kTileCost[R > 1][i] * t.cj * t.ck * (share > 1.5 ? share : 1.5);
+    if (time >= t_best) continue;
+    t_best = time;
+    l.ntk = (int)ntj;
+    l.nseg = (int)nti;
+    l.sl = (int)(TH - 2 * H);
+    l.SK = (int)(TW - 2 * H);
+    block = dim3(64 * (unsigned)t.nw);
+    grid = dim3((unsigned)(nti * ntj));
+    fn = t.fn[k];
+  }
   return AN5D_OK;
 }
 
@@ -293,10 +371,8 @@ static int adjoint_enqueue(const AdjPlan& ap, const an5d_problem* p, const void*
   // checkpoint 0 = u0; every other slot gets u0's halo (forward launches write interiors only)
   e = hipMemcpy2DAsync(ckpt(0), P * esz, du0, g.D2 * esz, g.D2 * esz, g.D0, hipMemcpyDeviceToDevice, st);
   if (e != hipSuccess) return hip_fail(e, "hipMemcpy2DAsync(u0)");
-  for (int i = 1; i <= L; i++) {
-    e = ap.adj->halo(ckpt(0), ckpt(i), (int)g.D0, (int)g.D2, P, R, st);
-    if (e != hipSuccess) return hip_fail(e, "halo copy");
-  }
+  e = ap.adj->halo(ckpt(0), ckpt(1), (long long)(ap.grid_bytes / esz), L, (int)g.D0, (int)g.D2, P, R, st);
+  if (e != hipSuccess) return hip_fail(e, "halo copy");
   // forward: launch j advances [t0, t0+kf); the state at every multiple of
   // bt inside it goes to that block's checkpoint
   const long long slot_elems = (long long)(ap.grid_bytes / esz);
@@ -334,10 +410,27 @@ static int adjoint_enqueue(const AdjPlan& ap, const an5d_problem* p, const void*
     t0 = t1;
   }
   if (ms_fwd) (void)hipEventRecord(ev1, st);
+  // the launches of the two block sizes (the last block may be shorter)
+  struct Planned {
+    AdjLaunch l{};
+    dim3 grid, block;
+    AdjFn fn = nullptr;
+  } planned[2];
+  long long used = 0;  // gradient slots
+  for (int i = 0; i < 2; i++) {
+    Planned& q = planned[i];
+    rc = adj_launch_plan(ap, i ? ap.blocks.back() : ap.blocks[0], q.l, q.grid, q.block, q.fn);
+    if (rc) return rc;
+    if (!q.fn) return fail(AN5D_E_UNSUPPORTED, "no adjoint kernel for this block size");
+    const long long n = (long long)q.l.ntk * q.l.nseg;
+    if (n > used) used = n;
+  }
+  if (used > ap.nslots) return fail(AN5D_E_INVALID, "workspace too small");
   // seed: lambda_T = u_T - target on the interior (0 on the halo), loss slots
   {
-    const long long nz = (long long)(ap.ws_bytes - ap.gslot_off) / (long long)sizeof(double);
-    hipLaunchKernelGGL(zero_f64_kernel, dim3(256), dim3(256), 0, st, gslot, nz);
+    const long long nz = used * ap.ng;
+    const long long blocks = cdiv(nz, 256);
+    hipLaunchKernelGGL(zero_f64_kernel, dim3((unsigned)(blocks < 256 ? blocks : 256)), dim3(256), 0, st, gslot, nz);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "slot clear");
   }
@@ -346,11 +439,8 @@ static int adjoint_enqueue(const AdjPlan& ap, const an5d_problem* p, const void*
   // reverse blocks
   int cur = 0;
   for (int i = L - 1; i >= 0; i--) {
-    const int k = ap.blocks[i];
-    AdjLaunch l{};
-    dim3 grid, block;
-    rc = adj_launch_plan(ap, k, l, grid, block);
-    if (rc) return rc;
+    const Planned& q = planned[ap.blocks[i] == ap.blocks[0] ? 0 : 1];
+    AdjLaunch l = q.l;
     l.U = ckpt(i);
     l.Lin = lam[cur];
     l.Lout = lam[cur ^ 1];
@@ -358,15 +448,14 @@ static int adjoint_enqueue(const AdjPlan& ap, const an5d_problem* p, const void*
     l.gscale = gscale;
     l.has_div = has_div;
     l.gslot = gslot;
-    if (!ap.adj->fn[k]) return fail(AN5D_E_UNSUPPORTED, "no adjoint kernel for this block size");
-    e = ap.adj->fn[k](l, grid, block, st);
+    e = q.fn(l, q.grid, q.block, st);
     if (e != hipSuccess) return hip_fail(e, "adjoint launch");
     cur ^= 1;
   }
   e = hipMemcpy2DAsync(dgrad, g.D2 * esz, lam[cur], P * esz, g.D2 * esz, g.D0,
                        hipMemcpyDeviceToDevice, st);
   if (e != hipSuccess) return hip_fail(e, "hipMemcpy2DAsync(grad)");
-  hipLaunchKernelGGL(adj_finish_kernel, dim3(ap.ng + 1), dim3(256), 0, st, gslot, ap.nslots, ap.ng,
+  hipLaunchKernelGGL(adj_finish_kernel, dim3(ap.ng + 1), dim3(256), 0, st, gslot, used, ap.ng,
                      dgcoef, lslot, kSeedBlocks * 4, dloss);
   e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "gradient reduction");
@@ -412,10 +501,6 @@ extern "C" int an5d_adjoint_device(const an5d_problem* p, const void* du0, const
 // address comes from hipGetSymbolAddress, once per device, and only that
 // address is passed to kernels.
 namespace an5d {
-
-constexpr size_t kNoAllocScratchBytes = 64ull << 20;
-constexpr size_t kNoAllocCoefBytes = 1024;  // >= (81 taps + 2) * 8 bytes
-static_assert(kNoAllocScratchBytes % 256 == 0, "scratch is carved in 256-byte units");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -105,8 +105,16 @@ struct AdjLaunch {
 using AdjFn = hipError_t (*)(const AdjLaunch&, dim3 grid, dim3 block, hipStream_t);
 using SeedFn = hipError_t (*)(const void* uT, const void* target, void* lam, double* lslot, int D0,
                               int D2, long long s0, long long st, int R, hipStream_t);
-using HaloFn = hipError_t (*)(const void* src, void* dst, int D0, int D2, long long s0, int R,
-                              hipStream_t);
+// copies src's halo cells into ndst grids, dst_stride elements apart
+using HaloFn = hipError_t (*)(const void* src, void* dst, long long dst_stride, int ndst, int D0, int D2,
+                              long long s0, int R, hipStream_t);
+
+// A register-tile form of the reverse block (adj_tile.hpp); ck == 0: none.
+struct AdjTile {
+  int ck, cj, nw;
+  AdjFn fn[kMaxBT + 1];
+};
+constexpr int kAdjTiles = 2;
 
 struct AdjVariant {
   int stencil, dtype;
@@ -115,6 +123,7 @@ struct AdjVariant {
   HaloFn halo;
   AdjFn fn[kMaxBT + 1];
   int (*occupancy)(int bt);  // resident workgroups per CU of fn[bt] (0: unknown)
+  AdjTile tile[kAdjTiles];  // small grids first
 };
 
 std::vector<AdjVariant>& adj_registry();

@@ -66,6 +66,7 @@ FIELDS = {
     "plane_kernel": ["bt", "ck", "cj", "nw", "exact"],
     "direct_kernel": ["ck", "exact"],
     "adjoint_kernel": ["bt", "ck", "nw"],
+    "adjoint_tile_kernel": ["bt", "ck", "cj", "nw"],
     "rows_kernel": ["ck", "nw", "exact"],
     "rows_kernel_cap": ["ck", "nw", "exact", "waves_per_eu"],
     "rows3_kernel": ["ck", "cj", "nw", "exact"],

@@ -205,6 +205,33 @@ def test_adjoint_workspace_beyond_device_memory_is_rejected(torch_cuda):
         pyan5d.AdjointWorkspace("j2d5pt", [16384, 16384], 20000, np.float32, bt=1)
 
 
+@pytest.mark.parametrize("name", ["star2d1r", "star2d2r", "star2d3r", "star2d4r", "box2d1r", "box2d2r", "j2d5pt",
+                                  "j2d9pt", "j2d9pt-gol"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_adjoint_small_grids_at_tile_edges(name, dt):
+    """Small FP64 grids take the register tiles (64 to 256 columns by 16 to 64
+    rows): one cell, one tile, a cell more in either direction, several tiles,
+    with a short last block; against the FP64 oracle and against the streamed
+    kernel (an explicit segment length).  FP32 streams both times."""
+    r = O.info(name)["rad"]
+    tw = 64 if r == 1 else 128 if r == 2 else 256
+    bt = adj_btmax(name, dt)
+    T = 2 * bt + 1
+    tol = 1e-10 if dt == np.float64 else 2e-4
+    for n in ([1, 1], [32 - 2 * r, tw - 2 * r], [33 - 2 * r, tw - 2 * r], [32 - 2 * r, tw + 1 - 2 * r], [150, 310]):
+        u0, target, c, div = problem(name, n, dt, seed=sum(n))
+        print(f"case adjoint tiles {name} {np.dtype(dt).name} n={n}", flush=True)
+        loss, g, gc, _, _ = pyan5d.adjoint_host(name, u0, target, n, T, coefs=c, divisor=div)
+        sloss, sg, sgc, _, _ = pyan5d.adjoint_host(name, u0, target, n, T, coefs=c, divisor=div, sl=16)
+        oloss, og, ogc = O.adjoint(name, u0.astype(np.float64), target.astype(np.float64), n, T, coefs=c,
+                                   divisor=div)
+        assert loss == sloss
+        for a, b, o in ((g, sg, og), (gc, sgc, ogc)):
+            scale = max(1e-30, np.max(np.abs(o)))
+            assert np.max(np.abs(a - o)) <= tol * scale
+            assert np.max(np.abs(b - o)) <= tol * scale
+
+
 @pytest.mark.parametrize("n", [[700, 900], [2000, 1500]])
 def test_adjoint_block_deeper_than_the_tuned_forward_kernel(n):
     """Where the tuned forward choice is a one-step kernel (the wide boxes), the
