@@ -113,7 +113,7 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
   if (p->timesteps < 1) return fail(AN5D_E_INVALID, "adjoint needs timesteps >= 1");
   ap.adj = adj_variant(p->stencil, p->dtype);
   if (!ap.adj) return fail(AN5D_E_UNSUPPORTED, "no adjoint kernels for this stencil/dtype");
-  auto vs = variants_of(p->stencil, p->dtype);
+  const auto& vs = variants_of(p->stencil, p->dtype);
   if (cfg && cfg->variant >= (int)vs.size()) return fail(AN5D_E_INVALID, "variant index out of range");
   // forward kernel: the caller's variant, else the tuned/default forward choice
   an5d_config fc{0, cfg ? cfg->variant : -1, 0, AN5D_EXACT};

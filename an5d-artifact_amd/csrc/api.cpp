@@ -70,11 +70,16 @@ std::vector<Variant>& registry() {
   return v;
 }
 
-std::vector<const Variant*> variants_of(int stencil, int dtype) {
-  std::vector<const Variant*> out;
-  for (const Variant& v : registry())
-    if (v.stencil == stencil && v.dtype == dtype) out.push_back(&v);
-  return out;
+const std::vector<const Variant*>& variants_of(int stencil, int dtype) {
+  // indexed once: a scan of the registry costs more than a kernel launch
+  static const std::vector<std::vector<const Variant*>> table = [] {
+    std::vector<std::vector<const Variant*>> t(2 * kNumStencils);
+    for (const Variant& v : registry()) t[2 * v.stencil + (v.dtype == kF64)].push_back(&v);
+    return t;
+  }();
+  static const std::vector<const Variant*> none;
+  if (stencil < 0 || stencil >= kNumStencils || (dtype != kF32 && dtype != kF64)) return none;
+  return table[2 * stencil + (dtype == kF64)];
 }
 
 const StencilRT& stencil_rt(int id) {
@@ -462,7 +467,7 @@ int default_bt(const StencilRT& s, int dtype) {
 
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,
             int* slout) {
-  auto vs = variants_of(p->stencil, p->dtype);
+  const auto& vs = variants_of(p->stencil, p->dtype);
   if (vs.empty()) return fail(AN5D_E_UNSUPPORTED, "no kernels compiled for this stencil/dtype");
   const StencilRT& s = stencil_rt(p->stencil);
   int want_bt = cfg ? cfg->bt : 0;
@@ -525,7 +530,7 @@ extern "C" int an5d_resolve_config(const an5d_problem* p, const an5d_config* cfg
   if (rc) return rc;
   LaunchPlan lp;
   if (!plan_launch(*v, bt, g, sl, lp, err, rcfg.mode)) return fail(AN5D_E_UNSUPPORTED, err);
-  auto vs = variants_of(p->stencil, p->dtype);
+  const auto& vs = variants_of(p->stencil, p->dtype);
   int vi = 0;
   while (vi < (int)vs.size() && vs[vi] != v) vi++;
   *out = an5d_config{bt, vi, v->kind == kDirect ? 0 : lp.args.sl, mode};
@@ -607,7 +612,7 @@ extern "C" int an5d_variant_count(int stencil, int dtype) {
 }
 
 extern "C" int an5d_variant_get_info(int stencil, int dtype, int variant, an5d_variant_info* out) {
-  auto vs = variants_of(stencil, dtype);
+  const auto& vs = variants_of(stencil, dtype);
   if (variant < 0 || variant >= (int)vs.size() || !out) return fail(AN5D_E_INVALID, "bad variant");
   const Variant* v = vs[variant];
   out->kind = v->kind; out->ck = v->ck; out->cj = v->cj; out->nw = v->nw;

@@ -193,7 +193,7 @@ using namespace an5d;
 
 extern "C" int an5d_model_estimate(const an5d_problem* p, const an5d_config* cfg, double* gstencil) {
   if (!p || !cfg || !gstencil) return fail(AN5D_E_INVALID, "null argument");
-  auto vs = variants_of(p->stencil, p->dtype);
+  const auto& vs = variants_of(p->stencil, p->dtype);
   if (cfg->variant < 0 || cfg->variant >= (int)vs.size()) return fail(AN5D_E_INVALID, "bad variant");
   *gstencil = model_gstencil(p, *vs[cfg->variant], cfg->bt, cfg->sl, cfg->mode);
   return AN5D_OK;
@@ -206,7 +206,7 @@ extern "C" int an5d_autotune(const an5d_problem* p, void* dA, const an5d_layout*
   if (!make_geom(p, g, err)) return fail(AN5D_E_INVALID, err);
   if (mode != AN5D_EXACT && mode != AN5D_FAST) return fail(AN5D_E_INVALID, "bad mode");
   if (max_measured <= 0) max_measured = 24;
-  auto vs = variants_of(p->stencil, p->dtype);
+  const auto& vs = variants_of(p->stencil, p->dtype);
   if (vs.empty()) return fail(AN5D_E_UNSUPPORTED, "no kernels for this stencil/dtype");
   struct Cand {
     int variant, bt, sl;
@@ -376,7 +376,7 @@ extern "C" int an5d_tune_save(const char* path) {
   fprintf(f, "# stencil dtype mode n0 n1 n2 variant bt sl gstencil_per_s regcap (autotuner results; regcap:\n"
              "# registers per lane the chosen kernel was compiled to, 0 = no cap; informational)\n");
   for (const Entry& e : t.rows) {
-    auto vs = variants_of(e.stencil, e.dtype);
+    const auto& vs = variants_of(e.stencil, e.dtype);
     const int cap = e.variant >= 0 && e.variant < (int)vs.size() && e.bt * 2 > vs[e.variant]->btmax
                         ? vs[e.variant]->regcap
                         : 0;

@@ -442,7 +442,7 @@ int init_inst(const an5d_problem* p, int i, Inst& I) {
 // kernel's shape (CK = 4, four independent waves) and the batch's default
 // segment length ranks bt = 1 .. kBatchMaxBT.
 int prior_bt(const an5d_problem* p) {
-  auto vs = variants_of(p->stencil, p->dtype);
+  const auto& vs = variants_of(p->stencil, p->dtype);
   const Variant* v = nullptr;
   for (const Variant* x : vs)
     if (x->kind == kSweep && x->ck == batch_ck() && x->nw == 4) v = x;

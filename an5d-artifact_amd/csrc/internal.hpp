@@ -37,7 +37,7 @@ struct TunedChoice {
 int fail(int code, const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
 const StencilRT& stencil_rt(int id);
-std::vector<const Variant*> variants_of(int stencil, int dtype);
+const std::vector<const Variant*>& variants_of(int stencil, int dtype);
 bool make_geom(const an5d_problem* p, Geom& g, std::string& err);
 an5d_layout reference_layout(const Geom& g);
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,

@@ -7,6 +7,7 @@ no CPU fallback: if the library is missing every entry point raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import sys
 
@@ -130,15 +131,22 @@ def _check(rc):
     return rc
 
 
+@functools.lru_cache(maxsize=None)
 def stencil_id(name: str) -> int:
     return _check(lib().an5d_stencil_id(name.encode()))
 
 
-def info(name):
+@functools.lru_cache(maxsize=None)
+def _info(name):
+    """The stencil's descriptor (constant; asked of the library once)."""
     st = StencilInfo()
     _check(lib().an5d_stencil_get_info(stencil_id(name), ctypes.byref(st)))
     return dict(name=st.name.decode(), dim=st.dim, rad=st.rad, fpp=st.fpp, ntaps=st.ntaps,
                 divisor=st.divisor, linear=bool(st.linear))
+
+
+def info(name):
+    return dict(_info(name))
 
 
 def stencil_names():
@@ -151,7 +159,7 @@ def stencil_names():
 
 
 def taps(name):
-    n = info(name)["ntaps"]
+    n = _info(name)["ntaps"]
     offs = (ctypes.c_int * (4 * n))()
     coefs = (ctypes.c_double * n)()
     _check(lib().an5d_stencil_taps(stencil_id(name), offs, coefs, n))
@@ -187,7 +195,7 @@ def _dtype_code(dt):
 
 def grid_extents(name, n):
     """Full extents (interior + halo) of one buffer for interior extents n."""
-    d = info(name)
+    d = _info(name)
     if len(n) != d["dim"]:
         raise ValueError(f"{name} is {d['dim']}D: n must have {d['dim']} extents, got {list(n)}")
     if any(int(x) < 1 for x in n):
@@ -248,7 +256,7 @@ def make_problem(name, n, T, dtype, coefs=None, divisor=-1.0):
     keep = None
     if coefs is not None:
         keep = np.ascontiguousarray(np.asarray(coefs, dtype=np.float64)).ravel()
-        d = info(name)
+        d = _info(name)
         want = d["ntaps"] if d["linear"] else 2
         if keep.size != want:
             raise ValueError(f"{name} takes {want} coefficients, got {keep.size}")
@@ -286,7 +294,7 @@ def cpu_forward(name, A, n, T, coefs=None, divisor=-1.0, threads=0):
 
 def kernel_stencil(name, A, compsize, T, scop=True):
     """The drop-in entry (common.h:42 signature) on a host array; returns ms."""
-    _check_host(A, name, [compsize] * info(name)["dim"], 2)
+    _check_host(A, name, [compsize] * _info(name)["dim"], 2)
     ms = ctypes.c_double()
     _check(lib().an5d_kernel_stencil(stencil_id(name), _dtype_code(A.dtype), A.ctypes.data,
                                      int(compsize), int(T), 1 if scop else 0, ctypes.byref(ms)))
@@ -296,7 +304,7 @@ def kernel_stencil(name, A, compsize, T, scop=True):
 def init_grid(name, n, dtype=np.float32, mode=0, seed_base=None):
     """Both buffers of a host grid for interior extents n: mode 0 is the
     reference's init_grid (seed i + compsize), mode 1 uniform [0, 1)."""
-    d = info(name)
+    d = _info(name)
     shape = (2,) + tuple(int(x) + 2 * d["rad"] for x in n)
     A = np.empty(shape, dtype=dtype)
     if seed_base is None:
@@ -327,7 +335,7 @@ def layout_of(t, dim):
 def forward_device(name, t, n, T, coefs=None, divisor=-1.0, bt=0, variant=-1, sl=0, stream=None,
                    mode=EXACT):
     """Enqueue T steps on a device tensor t[2, ...]; returns immediately."""
-    d = info(name)
+    d = _info(name)
     _check_pair(t, name, n)
     p, keep = make_problem(name, n, T, _np_dtype(t), coefs, divisor)
     cfg = make_config(bt, variant, sl, mode)
@@ -340,7 +348,7 @@ def forward_device(name, t, n, T, coefs=None, divisor=-1.0, bt=0, variant=-1, sl
 def launch(name, t, n, steps, c0=0, coefs=None, divisor=-1.0, bt=0, variant=-1, sl=0, stream=None,
            mode=EXACT):
     """One launch of `steps` fused steps from buffer c0%2 to (c0+1)%2."""
-    d = info(name)
+    d = _info(name)
     _check_pair(t, name, n)
     p, keep = make_problem(name, n, steps, _np_dtype(t), coefs, divisor)
     cfg = make_config(bt if bt else steps, variant, sl, mode)
@@ -367,7 +375,7 @@ def adjoint_host(name, u0, target, n, T, coefs=None, divisor=-1.0, bt=0, variant
     target = np.ascontiguousarray(target, dtype=u0.dtype)
     _check_host(u0, name, n, 0)
     _check_host(target, name, n, 0)
-    d = info(name)
+    d = _info(name)
     p, keep = make_problem(name, n, T, u0.dtype, coefs, divisor)
     cfg = make_config(bt, variant, sl)
     grad = np.zeros_like(u0)
@@ -401,7 +409,7 @@ def _check_adjoint_args(name, n, u0, target, grad, gcoef, loss):
     _check_device(u0, "u0", shape=ext, contiguous=True)
     _check_device(target, "target", shape=ext, dtype=u0.dtype, contiguous=True)
     _check_device(grad, "grad", shape=ext, dtype=u0.dtype, contiguous=True)
-    d = info(name)
+    d = _info(name)
     ng = d["ntaps"] if d["linear"] else 2
     _check_device(gcoef, "gcoef", shape=[ng], dtype=torch.float64, contiguous=True)
     _check_device(loss, "loss", dtype=torch.float64, contiguous=True)
@@ -538,7 +546,7 @@ def autotune(name, n, dtype=np.float32, mode=EXACT, max_measured=24, tensor=None
         if _np_dtype(tensor) != np.dtype(dtype):
             raise ValueError("tensor dtype differs from dtype")
         ptr = ctypes.c_void_p(tensor.data_ptr())
-        lay = ctypes.byref(layout_of(tensor, info(name)["dim"]))
+        lay = ctypes.byref(layout_of(tensor, _info(name)["dim"]))
     _check(lib().an5d_autotune(ctypes.byref(p), ptr, lay, int(mode), int(max_measured),
                                ctypes.byref(best), ctypes.byref(gs)))
     return dict(bt=best.bt, variant=best.variant, sl=best.sl, mode=best.mode), gs.value
