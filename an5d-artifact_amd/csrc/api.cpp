@@ -38,7 +38,7 @@ int hip_fail(hipError_t e, const char* what) {
   void register_variants_##id##_1(std::vector<Variant>&);
 AN5D_STENCILS(AN5D_DECL_REG)
 // cols_inst.hip, tile2_inst.hip: the stencils the Makefile builds them for
-#define AN5D_COLS_IDS(X) X(5) X(6) X(7) X(17) X(18) X(19)
+#define AN5D_COLS_IDS(X) X(5) X(6) X(7) X(16) X(20) X(17) X(18) X(19)
 #define AN5D_TILE_IDS(X) X(0) X(1) X(2) X(3) X(4) X(5) X(8) X(9) X(10) X(11)
 #define AN5D_DECL_COLS(id)                            \
   void register_cols_##id##_0(std::vector<Variant>&); \
@@ -655,7 +655,7 @@ int run_schedule(const an5d_problem* p, void* dA, const an5d_layout* layout,
     if (share && v->fn_share[k] && v->share_scratch[k] && v->share_scratch[k]() == 0) return kLaunchShare;
     return rcfg.mode;
   };
-  if (v->kind == kCols && g.dim == 3) cols_coefs(p, cbytes, rcfg.mode);
+  if (v->kind == kCols && g.dim == 3 && g.r > 1) cols_coefs(p, cbytes, rcfg.mode);
   const void* dcoef = nullptr;
   rc = device_coefs(cbytes, &dcoef);
   if (rc) return rc;

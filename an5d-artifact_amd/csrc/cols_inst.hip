@@ -1,6 +1,7 @@
 // Instantiates and registers the column kernels of one box x dtype
 // (-DAN5D_SID=<stencil id> -DAN5D_F64=<0|1>).
 #include "cols.hpp"
+#include "cols1.hpp"
 #include "cols2.hpp"
 #include "launch.hpp"
 
@@ -12,7 +13,8 @@ constexpr int SID = AN5D_SID;
 
 template <int CK, bool EXACT>
 constexpr auto cols_fn() {
-  if constexpr (Def<SID>::dim == 3) return &cols_kernel<SID, T, CK, EXACT>;
+  if constexpr (Def<SID>::dim == 3 && Def<SID>::rad == 1) return &cols1_kernel<SID, T, CK, EXACT>;
+  else if constexpr (Def<SID>::dim == 3) return &cols_kernel<SID, T, CK, EXACT>;
   else return &cols2_kernel<SID, T, CK, EXACT>;
 }
 
@@ -40,7 +42,11 @@ void add_cols(std::vector<Variant>& out) {
 #define AN5D_CAT2(a, b, c) a##b##_##c
 #define AN5D_CAT(a, b, c) AN5D_CAT2(a, b, c)
 void AN5D_CAT(register_cols_, AN5D_SID, AN5D_F64)(std::vector<Variant>& out) {
-  add_cols<4>(out);
+  // radius-1 3D: two cells a lane in FP64 (bound by memory: more waves) and for
+  // the smaller FP32 grids
+  constexpr bool narrow = Def<SID>::dim == 3 && Def<SID>::rad == 1;
+  if constexpr (!(narrow && AN5D_F64)) add_cols<4>(out);
+  if constexpr (narrow) add_cols<2>(out);
 }
 
 }  // namespace an5d

@@ -71,6 +71,7 @@ FIELDS = {
     "rows_kernel_cap": ["ck", "nw", "exact", "waves_per_eu"],
     "rows3_kernel": ["ck", "cj", "nw", "exact"],
     "cols_kernel": ["ck", "exact"],
+    "cols1_kernel": ["ck", "exact"],
     "cols2_kernel": ["ck", "exact"],
     "tile2_kernel": ["ck", "cj", "nw", "exact"],
 }

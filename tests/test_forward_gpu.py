@@ -453,3 +453,27 @@ def test_host_arrays_with_two_halos(name, n, dt):
         O.run(name, B, n, T)
         # the schedule may end with fewer launches than steps only for bt > 1
         assert same(A, B)
+
+
+@pytest.mark.parametrize("name", ["box3d1r", "j3d27pt"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_box3d1_column_kernel_ragged_grids(name, dt):
+    """The column kernel of the 27-point boxes (kind 4): one run per row, rows
+    that end inside a run, a nearly empty last workgroup, segments of one plane,
+    fewer than three and the default; with and without the division, and in FMA
+    mode within 1e-5 / 1e-12 of the field's largest value."""
+    for v in pyan5d.variants(name, 0 if dt == np.float32 else 1):
+        if v["kind"] != 4:
+            continue
+        for n, sl, div in [([1, 1, 4], 0, -1.0), ([5, 6, 7], 1, 7.0), ([9, 17, 66], 2, 159.0), ([12, 33, 31], 0, 0.0)]:
+            T = 4
+            print(f"case columns {name} {np.dtype(dt).name} variant {v['index']} n={n} sl={sl} divisor={div}",
+                  flush=True)
+            A = rand_grid(name, n, dt, seed=sum(n))
+            B, C = A.copy(), A.copy()
+            pyan5d.forward_host(name, A, n, T, variant=v["index"], sl=sl, divisor=div)
+            O.run(name, B, n, T, divisor=div)
+            assert same(A[T % 2], B[T % 2])
+            pyan5d.forward_host(name, C, n, T, variant=v["index"], sl=sl, divisor=div, mode=pyan5d.FAST)
+            got, ref = C[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
+            assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
