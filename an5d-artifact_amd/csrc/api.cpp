@@ -37,9 +37,14 @@ int hip_fail(hipError_t e, const char* what) {
   void register_variants_##id##_0(std::vector<Variant>&);     \
   void register_variants_##id##_1(std::vector<Variant>&);
 AN5D_STENCILS(AN5D_DECL_REG)
-// cols_inst.hip, tile2_inst.hip: the stencils the Makefile builds them for
+// cols_inst.hip, tile2_inst.hip, tile3_inst.hip: the stencils the Makefile builds them for
 #define AN5D_COLS_IDS(X) X(5) X(6) X(7) X(16) X(20) X(17) X(18) X(19)
 #define AN5D_TILE_IDS(X) X(0) X(1) X(2) X(3) X(4) X(5) X(8) X(9) X(10) X(11)
+#define AN5D_TILE3_IDS(X) X(12) X(16) X(20)
+#define AN5D_DECL_TILE3(id)                            \
+  void register_tile3_##id##_0(std::vector<Variant>&); \
+  void register_tile3_##id##_1(std::vector<Variant>&);
+AN5D_TILE3_IDS(AN5D_DECL_TILE3)
 #define AN5D_DECL_COLS(id)                            \
   void register_cols_##id##_0(std::vector<Variant>&); \
   void register_cols_##id##_1(std::vector<Variant>&);
@@ -63,8 +68,12 @@ std::vector<Variant>& registry() {
 #define AN5D_CALL_TILE(id)     \
   register_tile2_##id##_0(out); \
   register_tile2_##id##_1(out);
+#define AN5D_CALL_TILE3(id)     \
+  register_tile3_##id##_0(out); \
+  register_tile3_##id##_1(out);
     AN5D_COLS_IDS(AN5D_CALL_COLS)
     AN5D_TILE_IDS(AN5D_CALL_TILE)
+    AN5D_TILE3_IDS(AN5D_CALL_TILE3)
     return out;
   }();
   return v;
@@ -248,6 +257,17 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     // but the grid's own edges
     const long long TH = (long long)v.nw * v.cj, TW = 64LL * v.ck, H = (long long)bt * R;
     if (TH <= 2 * H || TW <= 2 * H) { err = "bt too deep for this variant's tile"; return false; }
+    if (g.dim == 3) {
+      const long long nti = cdiv(n0, v.planes);
+      const long long ntj = g.D1 > TH ? cdiv(g.D1 - 2 * H, TH - 2 * H) : 1;
+      const long long ntk = g.D2 > TW ? cdiv(g.D2 - 2 * H, TW - 2 * H) : 1;
+      if (nti * ntj >= (1LL << 31) || nti * ntj * ntk >= (1LL << 31)) { err = "grid too large"; return false; }
+      a.ntk = (int)ntk; a.ntj = (int)ntj; a.nseg = (int)nti; a.sl = v.planes;
+      a.SK = (int)(TW - 2 * H); a.SJ = (int)(TH - 2 * H);
+      lp.block = dim3(64 * v.nw);
+      lp.grid = dim3((unsigned)(nti * ntj * ntk));
+      return true;
+    }
     const long long nti = g.D0 > TH ? cdiv(g.D0 - 2 * H, TH - 2 * H) : 1;
     const long long ntk = g.D2 > TW ? cdiv(g.D2 - 2 * H, TW - 2 * H) : 1;
     if (nti * ntk >= (1LL << 31)) { err = "grid too large"; return false; }

@@ -146,8 +146,13 @@ double model_gstencil(const an5d_problem* p, const Variant& v, int bt, int sl, i
     ovi = (lp.args.sl + 0.5 * g.r) / lp.args.sl;
   } else if (v.kind == kTile) {
     ovk = lp.args.ntk * 64.0 * v.ck / nk;
-    ovi = lp.args.nseg * (double)v.nw * v.cj / n0;
-    waves = (double)lp.args.ntk * lp.args.nseg * v.nw;
+    if (g.dim == 3) {
+      ovj = lp.args.ntj * (double)v.nw * v.cj / nj;
+      ovi = lp.args.nseg * (double)(v.planes + bt) / n0;
+    } else {
+      ovi = lp.args.nseg * (double)v.nw * v.cj / n0;
+    }
+    waves = (double)lp.args.ntk * lp.args.ntj * lp.args.nseg * v.nw;
   } else if (v.kind == kPlane) {
     ovk = lp.args.ntk * 64.0 * v.ck / nk;
     ovj = lp.args.ntj * (double)v.nw * v.cj / nj;

@@ -36,7 +36,7 @@ inline hipError_t lds_opt_in(const void* kernel, size_t lds, std::atomic<int>* d
 // kCols: one step per launch, a column (3D) or run (2D) of cells per lane, for
 // the boxes of radius >= 2; in 3D its coefficient table has an order of its own
 // (cols_coefs)
-// kTile: several steps per launch on a 2D tile held in registers
+// kTile: several steps per launch on a tile held in registers
 enum KernelKind { kSweep = 0, kDirect = 1, kPlane = 2, kRows = 3, kCols = 4, kTile = 5 };
 enum DType { kF32 = 0, kF64 = 1 };
 
@@ -65,6 +65,7 @@ struct Variant {
   int stencil, dtype, kind;
   int ck, cj, nw, btmax;
   int regcap;              // register cap per lane of the deeper blocks (0: none)
+  int planes;              // 3D register tiles: planes a tile owns
   size_t lds[kMaxBT + 1];  // dynamic LDS bytes per workgroup, by bt
   LaunchFn fn[kMaxBT + 1];       // fn[bt], bt in [1, btmax], exact mode
   LaunchFn fn_fast[kMaxBT + 1];  // fast (FMA) mode, same shapes

@@ -74,6 +74,7 @@ FIELDS = {
     "cols1_kernel": ["ck", "exact"],
     "cols2_kernel": ["ck", "exact"],
     "tile2_kernel": ["ck", "cj", "nw", "exact"],
+    "tile3_kernel": ["bt", "planes", "ck", "cj", "nw", "exact"],
 }
 
 

@@ -477,3 +477,23 @@ def test_box3d1_column_kernel_ragged_grids(name, dt):
             pyan5d.forward_host(name, C, n, T, variant=v["index"], sl=sl, divisor=div, mode=pyan5d.FAST)
             got, ref = C[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
             assert np.max(np.abs(got - ref)) <= (1e-5 if dt == np.float32 else 1e-12) * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("name", ["star3d1r", "box3d1r", "j3d27pt"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_3d_register_tiles_at_their_edges(name, dt):
+    """The 3D register tiles (kind 5: 8 planes of 32 rows x 64 cells): a grid of
+    one cell, of exactly one tile, a plane, row or cell more, several tiles, at
+    every depth; bit for bit the oracle."""
+    for v in pyan5d.variants(name, 0 if dt == np.float32 else 1):
+        if v["kind"] != 5:
+            continue
+        for bt in range(1, v["btmax"] + 1):
+            for n in ([1, 1, 1], [8, 30, 62], [9, 30, 62], [8, 31, 62], [8, 30, 63], [19, 61, 130]):
+                T = bt + 1
+                print(f"case tiles {name} {np.dtype(dt).name} variant {v['index']} bt={bt} n={n}", flush=True)
+                A = rand_grid(name, n, dt, seed=sum(n) + bt)
+                B = A.copy()
+                pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt)
+                O.run(name, B, n, T)
+                assert same(A[T % 2], B[T % 2])
