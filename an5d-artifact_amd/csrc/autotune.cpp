@@ -316,7 +316,7 @@ extern "C" int an5d_autotune(const an5d_problem* p, void* dA, const an5d_layout*
     if (rc) break;
     int reps = 2;
     double sec = 0.0;
-    for (int attempt = 0; attempt < 6; attempt++) {
+    for (;;) {
       (void)hipEventRecord(e0, nullptr);
       for (int r = 0; r < reps && rc == AN5D_OK; r++) rc = an5d_launch(&q, buf, &L, &cfg, c.bt, r, nullptr);
       (void)hipEventRecord(e1, nullptr);
@@ -325,7 +325,7 @@ extern "C" int an5d_autotune(const an5d_problem* p, void* dA, const an5d_layout*
       float ms = 0.f;
       (void)hipEventElapsedTime(&ms, e0, e1);
       sec = ms / 1e3;
-      if (sec > 2e-3) break;
+      if (sec > 2e-3 || reps >= 256) break;
       reps *= 2;
     }
     if (rc) break;

@@ -18,8 +18,15 @@
 // 10.6.  From 4096^2 on the streams of the radius-1 stencils win.
 // Shapes (tile2_inst.hip): 64 x 32 cells (few per lane, most workgroups) for the
 // smallest grids, 128 x 64 on 16 or 8 waves above; radius 3-4 needs four cells
-// a lane (256 wide).  Tried: 64 x 32 on 8 waves, 64 x 64, 128 x 32 (within 5 %
-// of a kept shape or slower everywhere).
+// a lane (256 wide).  FP32 also has 128 x 128 on 16 waves, which computes 1.2-1.5
+// cells per stored one where 128 x 64 computes 1.4-2, and 256 x 64 on 8, which
+// moves half as many cells between lanes: the first is best where one or two of
+// its tiles fill each CU (j2d9pt-gol FMA 1000x3001, one step: 2.78 -> 2.16 us,
+// 6144^2 20.1 -> 16.4; star2d2r 1000x3001 4.25 -> 4.02), the second from 6144^2
+// (j2d5pt FMA 8192^2 20.9 -> 20.2 us).  Tried: 64 x 32 on 8 waves, 64 x 64, 128 x
+// 32 (within 5 % of a kept shape or slower everywhere); resident workgroups that
+// take tiles in turn and load the next one's cells under this one's steps (8
+// waves 13-18 % slower at 4096^2 and 8192^2, 16 waves 5-8 % faster).
 #pragma once
 
 #include "engine.hpp"
@@ -43,67 +50,92 @@ constexpr size_t tile2_buf_bytes() {
 template <int ID, typename T, int CK, int CJ, int NW>
 constexpr int tile2_bufs() { return 2 * tile2_buf_bytes<ID, T, CK, CJ, NW>() <= 160 * 1024 ? 2 : 1; }
 
-template <int ID, typename T, int CK, int CJ, int NW, bool EXACT, int DM>
-__device__ __forceinline__ void tile2_body(const SweepArgs<T>& a) {
-  using D = Def<ID>;
-  constexpr int R = D::rad;
-  constexpr int NT = D::linear ? D::ntaps : 1;
-  constexpr int W = 64 * CK, TH = NW * CJ;
-  constexpr int ER = edge_rows<CJ, R>();
-  constexpr int NB = tile2_bufs<ID, T, CK, CJ, NW>();
-  static_assert(CK >= R, "a lane must hold at least R cells");
-  extern __shared__ __align__(16) unsigned char an5d_lds[];
-  T* const lds = reinterpret_cast<T*>(an5d_lds);
-
-  const int steps = a.steps, H = steps * R;
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b = xcd_tile(blockIdx.x, gridDim.x);
-  const int ti = b / a.ntk, tk = b - ti * a.ntk;
-  // the tile's first row and column in the grid, and what it owns
-  const int r0 = ti * a.SJ, c0 = tk * a.SK;
-  const bool top = ti == 0, bot = ti == a.nseg - 1;
-  const int olo = top ? R : r0 + H, ohi = bot ? a.D0 - R : r0 + TH - H;
-  const int klo = tk == 0 ? R : c0 + H, khi = tk == a.ntk - 1 ? a.D2 - R : c0 + W - H;
-  const int rw = r0 + w * CJ;        // the wave's first row
-  const int kl = c0 + lane * CK;     // the lane's first column
-
-  bool kin[CK], kst[CK], cells_in = true, kst_all = true;
+// Where a wave's part of a tile lies: its first row, the lane's first column,
+// the rows and columns the tile owns, and the wave's last step.
+template <int CK, int CJ, int NW>
+struct Tile2Pos {
+  int rw, kl, olo, ohi, last;
+  bool kin[CK], kst[CK], kst_all, wave_in;
+  __device__ __forceinline__ Tile2Pos(int R, int D0, int D2, int ntk, int nseg, int SJ, int SK, int tile, int steps,
+                                      int lane, int w) {
+    constexpr int W = 64 * CK, TH = NW * CJ;
+    const int H = steps * R;
+    const int ti = tile / ntk, tk = tile - ti * ntk;
+    const int r0 = ti * SJ, c0 = tk * SK;
+    const bool top = ti == 0, bot = ti == nseg - 1;
+    rw = r0 + w * CJ;
+    kl = c0 + lane * CK;
+    olo = top ? R : r0 + H;
+    ohi = bot ? D0 - R : r0 + TH - H;
+    // a row that stays exact: R rows are lost per step from every tile edge
+    // that is not the grid's
+    last = min(top ? steps : (w * CJ + CJ - 1) / R, bot ? steps : (TH - w * CJ - 1) / R);
+    const int klo = tk == 0 ? R : c0 + H, khi = tk == ntk - 1 ? D2 - R : c0 + W - H;
+    bool cells_in = true;
+    kst_all = true;
 #pragma unroll
-  for (int kk = 0; kk < CK; kk++) {
-    const int k = kl + kk;
-    kin[kk] = k >= R && k < a.D2 - R;
-    kst[kk] = k >= klo && k < khi;
-    cells_in = cells_in && kin[kk];
-    kst_all = kst_all && kst[kk];
-  }
-  const bool wave_in = __builtin_amdgcn_ballot_w64(!cells_in) == 0 && rw >= R && rw + CJ <= a.D0 - R;
-
-  T c[NT + 2];
-#pragma unroll
-  for (int q = 0; q < NT + 2; q++) c[q] = a.coef[q];
-  const T div = c[NT];
-  const int has_div = a.has_div;
-  const double gscale = a.gscale;
-
-  T u[CJ][CK];
-  if (c0 + W <= a.D2) {
-#pragma unroll
-    for (int jj = 0; jj < CJ; jj++) {
-      const int r = min(rw + jj, a.D0 - 1);
-      load_run<T, CK>(u[jj], a.src + (long long)r * a.s0 + kl);
+    for (int kk = 0; kk < CK; kk++) {
+      const int k = kl + kk;
+      kin[kk] = k >= R && k < D2 - R;
+      kst[kk] = k >= klo && k < khi;
+      cells_in = cells_in && kin[kk];
+      kst_all = kst_all && kst[kk];
     }
+    wave_in = __builtin_amdgcn_ballot_w64(!cells_in) == 0 && rw >= R && rw + CJ <= D0 - R;
+  }
+};
+
+// The lane's cells of a tile, rows and columns clamped into the grid.
+template <typename T, int CK, int CJ>
+__device__ __forceinline__ void tile2_load(T (&d)[CJ][CK], const T* src, long long s0, int D0, int D2, int ntk, int SJ,
+                                           int SK, int tile, int lane, int w) {
+  const int ti = tile / ntk, c0 = (tile - ti * ntk) * SK;
+  const int rw = ti * SJ + w * CJ, kl = c0 + lane * CK;
+  if (c0 + 64 * CK <= D2) {
+#pragma unroll
+    for (int jj = 0; jj < CJ; jj++) load_run<T, CK>(d[jj], src + (long long)min(rw + jj, D0 - 1) * s0 + kl);
   } else {
 #pragma unroll
     for (int jj = 0; jj < CJ; jj++) {
-      const T* row = a.src + (long long)min(rw + jj, a.D0 - 1) * a.s0;
+      const T* row = src + (long long)min(rw + jj, D0 - 1) * s0;
 #pragma unroll
-      for (int kk = 0; kk < CK; kk++) u[jj][kk] = row[min(kl + kk, a.D2 - 1)];
+      for (int kk = 0; kk < CK; kk++) d[jj][kk] = row[min(kl + kk, D2 - 1)];
     }
   }
+}
 
-  auto publish = [&](int buf) {
-    T* o = lds + (size_t)buf * (NW * ER * W) + (size_t)w * ER * W + lane * CK;
+template <typename T, int CK, int CJ, class Pos>
+__device__ __forceinline__ void tile2_store(const T (&u)[CJ][CK], const Pos& p, T* dst, long long s0) {
+#pragma unroll
+  for (int jj = 0; jj < CJ; jj++) {
+    const int r = p.rw + jj;
+    if (r < p.olo || r >= p.ohi) continue;
+    T* row = dst + (long long)r * s0 + p.kl;
+    if (p.kst_all) {
+      gstore_run<false, T, CK>(row, u[jj]);
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < CK; kk++)
+        if (p.kst[kk]) row[kk] = u[jj][kk];
+    }
+  }
+}
+
+// All steps of one tile.
+template <int ID, typename T, int CK, int CJ, int NW, bool EXACT, int DM, class Pos>
+__device__ __forceinline__ void tile2_steps(T (&u)[CJ][CK], T* lds, const Pos& p,
+                                            const T (&c)[(Def<ID>::linear ? Def<ID>::ntaps : 1) + 2], int has_div,
+                                            double gscale, int D0, int steps, int lane, int w) {
+  using D = Def<ID>;
+  constexpr int R = D::rad;
+  constexpr int NT = D::linear ? D::ntaps : 1;
+  constexpr int W = 64 * CK;
+  constexpr int ER = edge_rows<CJ, R>();
+  constexpr int NB = tile2_bufs<ID, T, CK, CJ, NW>();
+  static_assert(CK >= R, "a lane must hold at least R cells");
+  const T div = c[NT];
+  auto publish = [&](int to) {
+    T* o = lds + (size_t)to * (NW * ER * W) + (size_t)w * ER * W + lane * CK;
 #pragma unroll
     for (int jj = 0; jj < CJ; jj++) {
       const int e = edge_index<CJ, R>(jj);
@@ -111,13 +143,10 @@ __device__ __forceinline__ void tile2_body(const SweepArgs<T>& a) {
     }
   };
   publish(0);
-  // the wave's last step with a row that stays exact: R rows are lost per step
-  // from every tile edge that is not the grid's
-  const int last = min(top ? steps : (w * CJ + CJ - 1) / R, bot ? steps : (TH - w * CJ - 1) / R);
 #pragma unroll 1
   for (int s = 1; s <= steps; s++) {
     __syncthreads();
-    const bool live = s <= last;
+    const bool live = s <= p.last;
     T x[CJ + 2 * R][CK + 2 * R];
     if (live) {
       const T* in = lds + (size_t)(NB == 2 ? (s - 1) & 1 : 0) * (NW * ER * W) + lane * CK;
@@ -177,7 +206,7 @@ __device__ __forceinline__ void tile2_body(const SweepArgs<T>& a) {
               if (!zero_or_normal(val[jj][kk])) val[jj][kk] = sum[jj][kk] / div;
         }
       }
-      if (wave_in) {
+      if (p.wave_in) {
 #pragma unroll
         for (int jj = 0; jj < CJ; jj++)
 #pragma unroll
@@ -185,27 +214,33 @@ __device__ __forceinline__ void tile2_body(const SweepArgs<T>& a) {
       } else {
 #pragma unroll
         for (int jj = 0; jj < CJ; jj++) {
-          const bool rin = rw + jj >= R && rw + jj < a.D0 - R;
+          const bool rin = p.rw + jj >= R && p.rw + jj < D0 - R;
 #pragma unroll
-          for (int kk = 0; kk < CK; kk++) u[jj][kk] = rin && kin[kk] ? val[jj][kk] : u[jj][kk];
+          for (int kk = 0; kk < CK; kk++) u[jj][kk] = rin && p.kin[kk] ? val[jj][kk] : u[jj][kk];
         }
       }
       if (s < steps) publish(NB == 2 ? s & 1 : 0);
     }
   }
+}
+
+template <int ID, typename T, int CK, int CJ, int NW, bool EXACT, int DM>
+__device__ __forceinline__ void tile2_body(const SweepArgs<T>& a) {
+  using D = Def<ID>;
+  constexpr int NT = D::linear ? D::ntaps : 1;
+  extern __shared__ __align__(16) unsigned char an5d_lds[];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  T c[NT + 2];
 #pragma unroll
-  for (int jj = 0; jj < CJ; jj++) {
-    const int r = rw + jj;
-    if (r < olo || r >= ohi) continue;
-    T* row = a.dst + (long long)r * a.s0 + kl;
-    if (kst_all) {
-      gstore_run<false, T, CK>(row, u[jj]);
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < CK; kk++)
-        if (kst[kk]) row[kk] = u[jj][kk];
-    }
-  }
+  for (int q = 0; q < NT + 2; q++) c[q] = a.coef[q];
+  const Tile2Pos<CK, CJ, NW> p(D::rad, a.D0, a.D2, a.ntk, a.nseg, a.SJ, a.SK, tile, a.steps, lane, w);
+  T u[CJ][CK];
+  tile2_load<T, CK, CJ>(u, a.src, a.s0, a.D0, a.D2, a.ntk, a.SJ, a.SK, tile, lane, w);
+  tile2_steps<ID, T, CK, CJ, NW, EXACT, DM>(u, reinterpret_cast<T*>(an5d_lds), p, c, a.has_div, a.gscale, a.D0,
+                                            a.steps, lane, w);
+  tile2_store<T, CK, CJ>(u, p, a.dst, a.s0);
 }
 
 template <int ID, typename T, int CK, int CJ, int NW, bool EXACT>
@@ -214,6 +249,7 @@ __global__ __launch_bounds__(64 * NW) void tile2_kernel(SweepArgs<T> a) {
     tile2_body<ID, T, CK, CJ, NW, EXACT, 0>(a);
   } else if constexpr (Def<ID>::divisor != 0) {
     if (a.has_div == 2) tile2_body<ID, T, CK, CJ, NW, EXACT, 2>(a);
+    else if (a.has_div == 0) tile2_body<ID, T, CK, CJ, NW, EXACT, 0>(a);  // no test per cell
     else tile2_body<ID, T, CK, CJ, NW, EXACT, -1>(a);
   } else {
     if (a.has_div == 0) tile2_body<ID, T, CK, CJ, NW, EXACT, 0>(a);

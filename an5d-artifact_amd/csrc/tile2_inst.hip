@@ -48,10 +48,18 @@ void AN5D_CAT(register_tile2_, AN5D_SID, AN5D_F64)(std::vector<Variant>& out) {
     add_tile2<1, 2, 16>(out);
     add_tile2<2, 4, 16>(out);
     add_tile2<2, 8, 8>(out);
+    if constexpr (!AN5D_F64) {
+      add_tile2<2, 8, 16>(out);
+      add_tile2<4, 8, 8>(out);
+    }
   } else if constexpr (R == 2) {
     add_tile2<2, 2, 16>(out);
     add_tile2<2, 4, 16>(out);
     add_tile2<2, 8, 8>(out);
+    if constexpr (!AN5D_F64) {
+      add_tile2<2, 8, 16>(out);
+      add_tile2<4, 8, 8>(out);
+    }
   } else {
     add_tile2<4, 2, 16>(out);
     if constexpr (!AN5D_F64) {

@@ -2,10 +2,11 @@
 
     python -m pyan5d.tune [--set bench|ladder|all] [--stencils A,B] [--out FILE] [--max-measured K]
 
-"ladder": every stencil, dtype and mode at sides of powers of two, so that a
-grid of any size has a row of about its own cell count (the library takes the
-nearest one within 8x; kernel and depth carry over, the segment length is
-chosen for the grid at hand).  "all" is both sets.
+"ladder": every stencil, dtype and mode at sides of powers of two and, up to
+the sizes where launches fill the chip many times over, one size between, so
+that a grid of any size has a row of about its own cell count (the library
+takes the nearest one within 8x; kernel and depth carry over, the segment
+length is chosen for the grid at hand).  "all" is both sets.
 
 For every (stencil, dtype, size, mode, run length) of the set, an5d_autotune
 ranks all (kernel shape, register cap, bt, sl) candidates with the analytic
@@ -51,7 +52,7 @@ BENCH = [
 ]
 
 
-LADDER_2D = [256, 512, 1024, 2048, 4096, 8192, 16384]
+LADDER_2D = [256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192, 16384]
 LADDER_3D = [64, 128, 256, 512]
 
 

@@ -497,3 +497,21 @@ def test_3d_register_tiles_at_their_edges(name, dt):
                 pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt)
                 O.run(name, B, n, T)
                 assert same(A[T % 2], B[T % 2])
+
+
+@pytest.mark.parametrize("name", ["j2d5pt", "j2d9pt", "j2d9pt-gol", "gradient2d"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_register_tiles_division_modes(name, dt):
+    """The register tiles' three division forms (none, the source's divisor, any
+    other) on a grid of a few tiles with remainders; bit for bit the oracle."""
+    for v in pyan5d.variants(name, 0 if dt == np.float32 else 1):
+        if v["kind"] != 5:
+            continue
+        for div in (0.0, 118.0, 7.0) if name != "gradient2d" else (-1.0,):
+            n, T = [v["nw"] * v["cj"] + 9, 64 * v["ck"] + 21], 5
+            print(f"case tile divisions {name} {np.dtype(dt).name} variant {v['index']} divisor={div}", flush=True)
+            A = rand_grid(name, n, dt, seed=3)
+            B = A.copy()
+            pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=3, divisor=div)
+            O.run(name, B, n, T, divisor=div)
+            assert same(A[T % 2], B[T % 2])
