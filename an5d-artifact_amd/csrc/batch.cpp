@@ -32,6 +32,7 @@ namespace an5d {
 // batch_inst.hip
 hipError_t batch_launch_level(int kind, const BatchRec* recs, const BatchUnit* units, int nunits,
                               int* counter, int grid, hipStream_t st);
+hipError_t batch_launch_tiles(const BatchRec* recs, const BatchUnit* units, int nunits, hipStream_t st);
 hipError_t batch_launch_reset(int* counters, int n, hipStream_t st);
 int batch_occupancy(int kind);
 int batch_kind_of(int stencil);
@@ -48,6 +49,10 @@ constexpr int kRowsPerUnit = 8;  // PREP / SEED / GRAD rows per work unit
 constexpr int kSlCandidates[] = {32, 64, 128, 256};
 constexpr int kMinBatchSl = 32;
 constexpr int kDefaultSl = 64;
+// forward batch: a launch's loads and stores in steps
+constexpr double kTileCost = 4.0;
+// at least a quarter of a tile's rows is its own
+constexpr int tile_max_bt(int r) { return kTileNW * kTileCJ * 3 / 8 / r < kMaxBT ? kTileNW * kTileCJ * 3 / 8 / r : kMaxBT; }
 
 long long cdiv(long long a, long long b) { return (a + b - 1) / b; }
 size_t round256(size_t x) { return (x + 255) / 256 * 256; }
@@ -59,7 +64,7 @@ struct Inst {
   std::vector<int> steps;  // forward batch: launch schedule; adjoint batch: blocks in time order
   int sl_fixed = 0;        // caller's sl (0: the batch-wide one)
   int bt_fixed = 0;        // forward batch: caller's bt (0: the batch-wide policy)
-  int bt_prior = 1;        // forward batch: the model prior's bt
+  int bt_prior = 1;        // forward batch: the depth of least cost (prior_bt)
   // adjoint batch: coarse stride C (blocks), coarse slots S = ceil(L / C);
   // workspace slots: coarse 0..S-1, u_T at S, fine 1..C-1 at S+1..S+C-1,
   // lambda at S+C and S+C+1
@@ -129,8 +134,7 @@ struct an5d_batch {
   int n = 0;
   int levels = 0;
   int sl = kDefaultSl;
-  int bt_policy = 0;  // forward batch, instances without a caller bt: 0 the model prior, k > 0 bt = k
-  int counters_cap = 0;  // levels the counter array holds
+  int bt_policy = 0;  // forward batch, instances without a caller bt: 0 each one's own, k > 0 bt = k
   std::vector<Inst> inst;
   // level tables: the records of level l start at rec_off[l], its units at
   // unit_off[l]: first the nfwd[l] units of the forward-class kernel, then the
@@ -139,7 +143,7 @@ struct an5d_batch {
   BatchUnit* d_units = nullptr;
   std::vector<long long> rec_off, unit_off;
   std::vector<int> nfwd, nadj;
-  int* d_counters = nullptr;  // two per level
+  int* d_counters = nullptr;  // adjoint batch: two per level
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipStream_t cap = nullptr;
@@ -164,6 +168,17 @@ void fwd_tiling(const Inst& I, int k, int sl, BatchRec& r) {
   r.ntk = (int)cdiv(nk, SK);
   r.sl = (int)s;
   r.nseg = (int)cdiv(n0, s);
+}
+
+// Register tiles of a forward batch (tile2.hpp): each gives up k*R cells on
+// every side that is not the grid's edge.
+void tile_tiling(const Inst& I, int k, BatchRec& r) {
+  constexpr long long TH = kTileNW * kTileCJ, TW = 64 * kTileCK;
+  const long long H = (long long)k * I.g.r;
+  r.sl = (int)(TH - 2 * H);
+  r.SK = (int)(TW - 2 * H);
+  r.nseg = (int)(I.g.D0 > TH ? cdiv(I.g.D0 - 2 * H, r.sl) : 1);
+  r.ntk = (int)(I.g.D2 > TW ? cdiv(I.g.D2 - 2 * H, r.SK) : 1);
 }
 
 // the adjoint sweep's tiling (adjoint.cpp adj_launch_plan): lane-aligned
@@ -233,7 +248,7 @@ bool level_recs(const an5d_batch* b, const Inst& I, int m, std::vector<BatchRec>
     r.dst = static_cast<char*>(I.dA) + (size_t)((m + 1) % 2) * gbytes;
     r.s0 = I.g.D2;
     r.bt = k;
-    fwd_tiling(I, k, sl, r);
+    tile_tiling(I, k, r);
     recs.push_back(r);
     return true;
   }
@@ -339,7 +354,8 @@ void place_chains(an5d_batch* b) {
   b->levels = S;
 }
 
-double rec_cost(const BatchRec& r) {
+double rec_cost(const an5d_batch* b, const BatchRec& r) {
+  if (!b->adjoint) return r.bt;  // tiles of one size
   const double cells = (double)r.sl * 64.0 * batch_ck();
   if (r.type == kUnitAdj) return 2.0 * cells * r.bt;
   if (r.type == kUnitFwd) return cells * r.bt;
@@ -372,8 +388,8 @@ int build_levels(an5d_batch* b) {
       if (!level_recs(b, I, m, lv, err)) return fail(AN5D_E_UNSUPPORTED, err);
     }
     // the most expensive records first: their tiles start before the cheap ones
-    std::stable_sort(lv.begin(), lv.end(), [](const BatchRec& x, const BatchRec& y) {
-      return rec_cost(x) > rec_cost(y);
+    std::stable_sort(lv.begin(), lv.end(), [&](const BatchRec& x, const BatchRec& y) {
+      return rec_cost(b, x) > rec_cost(b, y);
     });
     for (int pass = 0; pass < 2; pass++) {  // forward-class units, then adjoint units
       long long nu = 0;
@@ -382,7 +398,10 @@ int build_levels(an5d_batch* b) {
         const int rid = (int)(recs.size() - b->rec_off[l]);
         recs.push_back(r);
         const long long nt = (long long)r.ntk * r.nseg;
-        for (long long t = 0; t < nt; t++) units.push_back(BatchUnit{rid, (int)t});
+        // tiles by the XCD that runs them (workgroups go round-robin over 8):
+        // neighbours, which read each other's halo, share its L2
+        const long long q = b->adjoint ? 0 : nt / 8;
+        for (long long t = 0; t < nt; t++) units.push_back(BatchUnit{rid, (int)(t < 8 * q ? t % 8 * q + t / 8 : t)});
         nu += nt;
       }
       if (nu >= (1LL << 31)) return fail(AN5D_E_UNSUPPORTED, "too many work units in one level");
@@ -438,21 +457,17 @@ int init_inst(const an5d_problem* p, int i, Inst& I) {
   return device_coefs(cb, &I.coef);
 }
 
-// Forward batch, bt not given: the autotuner's model prior at the batch
-// kernel's shape (CK = 4, four independent waves) and the batch's default
-// segment length ranks bt = 1 .. kBatchMaxBT.
-int prior_bt(const an5d_problem* p) {
-  const auto& vs = variants_of(p->stencil, p->dtype);
-  const Variant* v = nullptr;
-  for (const Variant* x : vs)
-    if (x->kind == kSweep && x->ck == batch_ck() && x->nw == 4) v = x;
+// Forward batch, bt not given: the depth whose tiles cost least per step, a
+// launch counted as kTileCost steps more (its loads and stores).
+int prior_bt(const Inst& I) {
   int best = 1;
-  double best_g = -1.0;
-  for (int bt = 1; bt <= batch_max_bt(); bt++) {
-    if (!v || bt > v->btmax) break;
-    const double gs = model_gstencil(p, *v, bt, kDefaultSl, AN5D_EXACT);
-    if (gs > best_g) {
-      best_g = gs;
+  double best_c = 1e300;
+  for (int bt = 1; bt <= tile_max_bt(I.g.r); bt++) {
+    BatchRec r;
+    tile_tiling(I, bt, r);
+    const double c = (double)r.ntk * r.nseg * (bt + kTileCost) / bt;
+    if (c < best_c) {
+      best_c = c;
       best = bt;
     }
   }
@@ -460,24 +475,16 @@ int prior_bt(const an5d_problem* p) {
 }
 
 // Forward batch: every instance's launch schedule under the batch's bt
-// policy, the chains placed, the counters sized.
-int plan_forward(an5d_batch* b) {
+// policy, the chains placed.
+void plan_forward(an5d_batch* b) {
   for (Inst& I : b->inst) {
     int bt = I.bt_fixed > 0 ? I.bt_fixed : (b->bt_policy > 0 ? b->bt_policy : I.bt_prior);
-    if (bt > batch_max_bt()) bt = batch_max_bt();
+    if (bt > tile_max_bt(I.g.r)) bt = tile_max_bt(I.g.r);
     const int nl = an5d_schedule(I.T, bt, nullptr, 0);
     I.steps.resize(nl);
     an5d_schedule(I.T, bt, I.steps.data(), nl);
   }
   place_chains(b);
-  if (b->levels > b->counters_cap) {
-    (void)hipFree(b->d_counters);
-    b->d_counters = nullptr;
-    hipError_t e = hipMalloc(&b->d_counters, sizeof(int) * 2 * (b->levels > 0 ? b->levels : 1));
-    if (e != hipSuccess) return fail(AN5D_E_ALLOC, "hipMalloc(batch counters)");
-    b->counters_cap = b->levels;
-  }
-  return AN5D_OK;
 }
 
 }  // namespace
@@ -503,11 +510,11 @@ extern "C" int an5d_batch_create(an5d_batch** out, int n, const an5d_problem* pr
       return fail(AN5D_E_UNSUPPORTED, "batched bt is at most " + std::to_string(batch_max_bt()));
     }
     I.bt_fixed = bt;
-    I.bt_prior = bt > 0 ? bt : prior_bt(&probs[i]);
+    I.bt_prior = bt > 0 ? bt : prior_bt(I);
     I.sl_fixed = (cfgs && cfgs[i].sl > 0) ? cfgs[i].sl : 0;
   }
-  int rc = plan_forward(b);
-  if (rc == AN5D_OK) rc = build_levels(b);
+  plan_forward(b);
+  int rc = build_levels(b);
   if (rc) { batch_free(b); return rc; }
   *out = b;
   return AN5D_OK;
@@ -628,7 +635,6 @@ extern "C" int an5d_batch_adjoint_create(an5d_batch** out, int n, const an5d_pro
   place_chains(b);
   hipError_t e = hipMalloc(&b->d_counters, sizeof(int) * 2 * (b->levels > 0 ? b->levels : 1));
   if (e != hipSuccess) { batch_free(b); return fail(AN5D_E_ALLOC, "hipMalloc(batch counters)"); }
-  b->counters_cap = b->levels;
   e = hipDeviceSynchronize();
   if (e != hipSuccess) { batch_free(b); return hip_fail(e, "batch workspace clear"); }
   int rc = build_levels(b);
@@ -648,18 +654,18 @@ extern "C" int an5d_batch_run(an5d_batch* b, void* stream) {
   if (!b) return fail(AN5D_E_INVALID, "null batch");
   hipStream_t st = static_cast<hipStream_t>(stream);
   hipError_t e;
+  if (b->levels == 0) return AN5D_OK;  // no instance has steps to run
   if (!b->exec) {
     if (!b->cap) {
       e = hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking);
       if (e != hipSuccess) return hip_fail(e, "hipStreamCreate");
     }
-    const int kf = b->adjoint ? kLevelFwdMisc : kLevelFwd;
     const int cus = device_cus();
     auto resident = [&](int kind) {
       const int occ = batch_occupancy(kind);
       return occ > 0 && cus > 0 ? (long long)occ * cus : 2048LL;
     };
-    const long long res_f = resident(kf), res_a = resident(kLevelAdj);
+    const long long res_f = b->adjoint ? resident(kLevelFwdMisc) : 0, res_a = b->adjoint ? resident(kLevelAdj) : 0;
     auto grid_of = [](long long units, long long res) {
       long long g = cdiv(units, 4);  // four waves per workgroup, one unit each at first
       if (g > res) g = res;
@@ -667,13 +673,17 @@ extern "C" int an5d_batch_run(an5d_batch* b, void* stream) {
     };
     e = hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
-    hipError_t le = batch_launch_reset(b->d_counters, 2 * b->levels, b->cap);
+    hipError_t le = b->adjoint ? batch_launch_reset(b->d_counters, 2 * b->levels, b->cap) : hipSuccess;
     for (int l = 0; l < b->levels && le == hipSuccess; l++) {
       const BatchRec* recs = b->d_recs + b->rec_off[l];
       const BatchUnit* uf = b->d_units + b->unit_off[l];
       const BatchUnit* ua = uf + b->nfwd[l];
+      if (!b->adjoint) {
+        if (b->nfwd[l] > 0) le = batch_launch_tiles(recs, uf, b->nfwd[l], b->cap);
+        continue;
+      }
       if (b->nfwd[l] > 0)
-        le = batch_launch_level(kf, recs, uf, b->nfwd[l], b->d_counters + 2 * l, grid_of(b->nfwd[l], res_f),
+        le = batch_launch_level(kLevelFwdMisc, recs, uf, b->nfwd[l], b->d_counters + 2 * l, grid_of(b->nfwd[l], res_f),
                                 b->cap);
       if (le == hipSuccess && b->nadj[l] > 0)
         le = batch_launch_level(kLevelAdj, recs, ua, b->nadj[l], b->d_counters + 2 * l + 1,
@@ -696,7 +706,7 @@ extern "C" int an5d_batch_run(an5d_batch* b, void* stream) {
   return AN5D_OK;
 }
 
-// Measured choice of the batch-wide segment length: the candidates are timed
+// Measured choice of the depth or the segment length: the candidates are timed
 // on the whole level sequence (each replay rewrites the same outputs from
 // the same inputs), the fastest is kept.
 extern "C" int an5d_batch_tune(an5d_batch* b, int reps, int* best_sl, double* best_ms) {
@@ -726,17 +736,20 @@ extern "C" int an5d_batch_tune(an5d_batch* b, int reps, int* best_sl, double* be
   int best = b->sl, best_pol = b->bt_policy;
   double best_t = -1.0;
   int rc = AN5D_OK;
-  // forward batch: bt policy (the model prior per instance, or one bt for all)
-  // x segment length; the forward + adjoint batch keeps its blocks
+  // forward batch: bt policy (each instance's own, or one bt for all); the
+  // forward + adjoint batch keeps its blocks and tries segment lengths
   std::vector<int> policies = {b->bt_policy};
-  if (!b->adjoint) policies = {0, 3, 4, 5};
+  std::vector<int> sls(kSlCandidates, kSlCandidates + sizeof(kSlCandidates) / sizeof(int));
+  if (!b->adjoint) {
+    policies = {0, 4, 6, 8};
+    sls = {b->sl};
+  }
   for (int pol : policies)
-  for (int sl : kSlCandidates) {
+  for (int sl : sls) {
     b->sl = sl;
     if (!b->adjoint && pol != b->bt_policy) {
       b->bt_policy = pol;
-      rc = plan_forward(b);
-      if (rc) break;
+      plan_forward(b);
     }
     rc = build_levels(b);
     if (rc) break;
@@ -771,8 +784,7 @@ extern "C" int an5d_batch_tune(an5d_batch* b, int reps, int* best_sl, double* be
   b->sl = best;
   if (!b->adjoint && best_pol != b->bt_policy) {
     b->bt_policy = best_pol;
-    rc = plan_forward(b);
-    if (rc) return rc;
+    plan_forward(b);
   }
   rc = build_levels(b);
   if (rc) return rc;

@@ -11,7 +11,8 @@
 // a HIP graph.
 //
 // Unit types:
-//   FWD    one wave tile of a forward launch (the sweep of sweep.hpp)
+//   FWD    one wave tile of a forward launch (the sweep of sweep.hpp); in the
+//          forward batch one workgroup tile (tile2.hpp), no counter
 //   ADJ    one wave tile of a reverse block (the adjoint of adjoint.hpp)
 //   PREP   rows of the initial state copied into checkpoint slot 0, with the
 //          halo cells of those rows copied into every other slot (the sweeps
@@ -22,6 +23,7 @@
 #pragma once
 
 #include "adjoint.hpp"
+#include "tile2.hpp"
 
 namespace an5d {
 
@@ -37,7 +39,7 @@ struct BatchRec {
   int rows;     // PREP / SEED / GRAD: rows per unit
   long long s0;      // row pitch (elements) of the grids src / dst / aux (workspace or caller grid)
   long long s0_ref;  // PREP / SEED / GRAD: row pitch of the caller's grid
-  int ntk, nseg, sl, SK;  // FWD / ADJ tiling
+  int ntk, nseg, sl, SK;  // FWD / ADJ tiling (workgroup tiles: sl is the rows owned)
   const void* coef;
   const void* src;  // FWD input grid | ADJ checkpoint | PREP u0 | SEED u_T | GRAD lambda_0
   void* dst;        // FWD output grid | ADJ lambda out | PREP slot 0 | SEED lambda_T | GRAD caller's grad
@@ -57,7 +59,7 @@ struct BatchUnit {
 };
 
 // level kernel kinds (see batch_level_kernel)
-constexpr int kLevelFwd = 0, kLevelFwdMisc = 1, kLevelAdj = 2;
+constexpr int kLevelFwdMisc = 0, kLevelAdj = 1;
 
 // Stencils the batched kernels are built for (2D, FP32): forward CK = 4, the
 // adjoint at its own FP32 shape (CK = 4 for radius <= 2).
@@ -67,6 +69,8 @@ constexpr int kBatchMaxBT = 5;
 constexpr int kBatchCK = 4;
 constexpr int kBatchNW = 4;
 constexpr int kBatchAdjCK = 4;
+// tile of the forward batch (tile2.hpp)
+constexpr int kTileCK = 2, kTileCJ = 8, kTileNW = 8;
 // deepest adjoint block per kind: the level kernel holding every adjoint body
 // stays within 256 VGPRs (two waves per SIMD); j2d5pt's bt = 5 body alone
 // takes 246 and would push it past
@@ -237,10 +241,63 @@ __device__ __forceinline__ void batch_finish(const BatchRec& r) {
   if (lane == 0) *r.out_loss = s;
 }
 
-// Level kernels, each with its own register budget: KIND 0 runs FWD units
-// (the forward batch), KIND 1 the FWD, PREP, SEED, GRAD and FINISH units of
-// the forward + adjoint batch, KIND 2 its ADJ units.  Every wave leaves the
-// loop once the counter passes nunits.
+template <int K, int DM>
+__device__ __forceinline__ void batch_tile_steps(float (&u)[kTileCJ][kTileCK], float* lds,
+                                                 const Tile2Pos<kTileCK, kTileCJ, kTileNW>& p, const BatchRec& r,
+                                                 int lane, int w) {
+  constexpr int ID = kBatchIds[K], NC = Def<ID>::ntaps + 2;
+  const float* coef = static_cast<const float*>(r.coef);
+  float c[NC];
+#pragma unroll
+  for (int q = 0; q < NC; q++)
+    c[q] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, coef[q])));
+  tile2_steps<ID, float, kTileCK, kTileCJ, kTileNW, true, DM>(u, lds, p, c, r.has_div, 1.0, r.D0, r.bt, lane, w);
+}
+
+template <int K>
+__device__ __forceinline__ void batch_tile_dispatch(float (&u)[kTileCJ][kTileCK], float* lds,
+                                                    const Tile2Pos<kTileCK, kTileCJ, kTileNW>& p, const BatchRec& r,
+                                                    int lane, int w) {
+  if (r.has_div == 0) {
+    batch_tile_steps<K, 0>(u, lds, p, r, lane, w);
+    return;
+  }
+  if constexpr (Def<kBatchIds[K]>::divisor != 0)
+    if (r.has_div == 2) {
+      batch_tile_steps<K, 2>(u, lds, p, r, lane, w);
+      return;
+    }
+  batch_tile_steps<K, -1>(u, lds, p, r, lane, w);
+}
+
+// A level of the forward batch: one workgroup per register tile (tile2.hpp) of
+// every instance.  Bound by vector issue, as a launch of one large grid is.  On
+// the streamed sweep's wave tiles a level of 24 instances had one or two waves a
+// SIMD and stopped at five steps.
+__global__ __launch_bounds__(64 * kTileNW, 5) void batch_tile_kernel(const BatchRec* __restrict__ recs,
+                                                                  const BatchUnit* __restrict__ units) {
+  extern __shared__ __align__(16) unsigned char an5d_lds[];
+  float* const lds = reinterpret_cast<float*>(an5d_lds);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const BatchUnit wu = units[blockIdx.x];
+  const BatchRec r = recs[wu.rec];
+  const Tile2Pos<kTileCK, kTileCJ, kTileNW> p(r.R, r.D0, r.D2, r.ntk, r.nseg, r.sl, r.SK, wu.tile, r.bt, lane, w);
+  float u[kTileCJ][kTileCK];
+  tile2_load<float, kTileCK, kTileCJ>(u, static_cast<const float*>(r.src), r.s0, r.D0, r.D2, r.ntk, r.sl, r.SK,
+                                      wu.tile, lane, w);
+  switch (r.kind) {
+    case 0: batch_tile_dispatch<0>(u, lds, p, r, lane, w); break;
+    case 1: batch_tile_dispatch<1>(u, lds, p, r, lane, w); break;
+    case 2: batch_tile_dispatch<2>(u, lds, p, r, lane, w); break;
+    default: batch_tile_dispatch<3>(u, lds, p, r, lane, w); break;
+  }
+  tile2_store<float, kTileCK, kTileCJ>(u, p, static_cast<float*>(r.dst), r.s0);
+}
+
+// Level kernels of the forward + adjoint batch, each with its own register
+// budget: one runs its FWD, PREP, SEED, GRAD and FINISH units, the other its ADJ
+// units.  Every wave leaves the loop once the counter passes nunits.
 template <int KIND>
 __global__ __launch_bounds__(64 * kBatchNW) void batch_level_kernel(const BatchRec* __restrict__ recs,
                                                                     const BatchUnit* __restrict__ units,
@@ -268,7 +325,7 @@ __global__ __launch_bounds__(64 * kBatchNW) void batch_level_kernel(const BatchR
           case 2: batch_fwd_dispatch<2>(r, wu.tile); break;
           default: batch_fwd_dispatch<3>(r, wu.tile); break;
         }
-      } else if constexpr (KIND == kLevelFwdMisc) {
+      } else {
         if (r.type == kUnitPrep) batch_prep(r, wu.tile);
         else if (r.type == kUnitSeed) batch_seed(r, wu.tile);
         else if (r.type == kUnitGrad) batch_grad(r, wu.tile);

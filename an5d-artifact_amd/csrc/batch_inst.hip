@@ -1,13 +1,14 @@
 // Instantiates the batched level kernels (FP32, the stencils of kBatchIds).
 #define AN5D_BATCH_KERNELS
+#include <algorithm>
+
 #include "batch.hpp"
 
 namespace an5d {
 
 static const void* level_kernel(int kind) {
   if (kind == kLevelAdj) return reinterpret_cast<const void*>(&batch_level_kernel<kLevelAdj>);
-  if (kind == kLevelFwdMisc) return reinterpret_cast<const void*>(&batch_level_kernel<kLevelFwdMisc>);
-  return reinterpret_cast<const void*>(&batch_level_kernel<kLevelFwd>);
+  return reinterpret_cast<const void*>(&batch_level_kernel<kLevelFwdMisc>);
 }
 
 hipError_t batch_launch_level(int kind, const BatchRec* recs, const BatchUnit* units, int nunits,
@@ -15,12 +16,22 @@ hipError_t batch_launch_level(int kind, const BatchRec* recs, const BatchUnit* u
   if (kind == kLevelAdj)
     hipLaunchKernelGGL(batch_level_kernel<kLevelAdj>, dim3(grid), dim3(64 * kBatchNW), 0, st, recs, units,
                        nunits, counter);
-  else if (kind == kLevelFwdMisc)
+  else
     hipLaunchKernelGGL(batch_level_kernel<kLevelFwdMisc>, dim3(grid), dim3(64 * kBatchNW), 0, st, recs,
                        units, nunits, counter);
-  else
-    hipLaunchKernelGGL(batch_level_kernel<kLevelFwd>, dim3(grid), dim3(64 * kBatchNW), 0, st, recs, units,
-                       nunits, counter);
+  return hipGetLastError();
+}
+
+template <int K>
+constexpr size_t tile_lds() {
+  return tile2_bufs<kBatchIds[K], float, kTileCK, kTileCJ, kTileNW>() *
+         tile2_buf_bytes<kBatchIds[K], float, kTileCK, kTileCJ, kTileNW>();
+}
+
+hipError_t batch_launch_tiles(const BatchRec* recs, const BatchUnit* units, int nunits, hipStream_t st) {
+  constexpr size_t lds = std::max({tile_lds<0>(), tile_lds<1>(), tile_lds<2>(), tile_lds<3>()});
+  static_assert(lds <= 65536 && kBatchKinds == 4, "more LDS needs an opt-in");
+  hipLaunchKernelGGL(batch_tile_kernel, dim3(nunits), dim3(64 * kTileNW), lds, st, recs, units);
   return hipGetLastError();
 }
 

@@ -214,15 +214,17 @@ int an5d_adjoint_host(const an5d_problem* prob, const void* u0, const void* targ
  * star2d2r and j2d9pt-gol; any sizes and timesteps.
  *
  * Each instance's work is a chain of levels; one kernel launch covers one
- * level of every instance, its waves pulling (instance, tile) work units of
- * every kind from a device counter, and the whole level sequence is captured
- * into one HIP graph on the first run (replayed afterwards).  Chains are
- * placed on the level axis so that the estimated work per level is even.
+ * level of every instance: a workgroup per tile in the forward batch, waves
+ * pulling (instance, tile) work units from a device counter in the forward +
+ * adjoint batch.  The whole level sequence is captured into one HIP graph on
+ * the first run (replayed afterwards).  Chains are placed on the level axis so
+ * that the estimated work per level is even.
  *
  * an5d_batch_create: forward only.  dA[i] holds both buffers of instance i
  * (reference layout); after a run buffer T_i%2 holds u_T, bit for bit the
- * single-grid result.  cfgs (optional): per-instance bt (<= 5; 0: ranked by
- * the autotuner's model at the batch kernel's shape) and sl (0: batch-wide).
+ * single-grid result.  cfgs (optional): per-instance bt (<= 5; 0: the
+ * depth of least cost for the instance's tiles) and sl (accepted; the forward
+ * batch has no segments).
  *
  * an5d_batch_adjoint_create: forward + adjoint.  Currently switched off: it
  * returns AN5D_E_UNSUPPORTED (its first GPU run stalled; cause not found).
@@ -239,10 +241,10 @@ int an5d_adjoint_host(const an5d_problem* prob, const void* u0, const void* targ
  * 3 for the radius-2 stars) and sl.  Loss and gradient sums are reduced in a
  * fixed order, so repeated runs give identical results.
  *
- * an5d_batch_tune: times the level sequence (`reps` replays each) at each
- * candidate batch-wide segment length (32-256) and, for a forward batch, bt
- * policy (each instance's model-prior bt, or bt = 3, 4, 5 for all instances
- * without a caller bt), and keeps the fastest; a forward batch's grids are
+ * an5d_batch_tune: times the level sequence (`reps` replays each) and keeps the
+ * fastest: for a forward batch over bt policies (each instance's own bt, or
+ * bt = 4, 6, 8 for all instances without a caller bt), for a forward + adjoint
+ * batch over batch-wide segment lengths (32-256); a forward batch's grids are
  * restored afterwards.  an5d_batch_run: enqueue one run on
  * `stream` (a hipStream_t); runs that overlap on one batch race. */
 typedef struct an5d_batch an5d_batch;

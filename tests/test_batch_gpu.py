@@ -258,3 +258,31 @@ def test_batch_adjoint_entry_is_switched_off(torch_cuda):
     with pytest.raises(pyan5d.An5dError) as e:
         pyan5d.BatchAdjoint(items)
     assert e.value.code == -2 and "switched off" in str(e.value)
+
+
+@pytest.mark.parametrize("bt", [0, 1, 5])
+def test_batch_tiles_at_their_edges(torch_cuda, bt):
+    """The batch's workgroup tiles (64 rows x 128 cells): one cell, exactly one
+    tile, a row or a cell more, one row or column of cells over many tiles;
+    every division form; each instance bit for bit the oracle."""
+    torch = torch_cuda
+    rng = np.random.default_rng(17)
+    items, hosts = [], []
+    for k, (name, div) in enumerate([("j2d5pt", 118.0), ("j2d5pt", 0.0), ("j2d9pt", 118.0), ("j2d9pt", 0.0),
+                                     ("star2d2r", -1.0), ("star2d2r", 3.0), ("j2d9pt-gol", 7.0)]):
+        r = O.info(name)["rad"]
+        for n in ([1, 1], [64 - 2 * r, 128 - 2 * r], [65 - 2 * r, 128 - 2 * r], [64 - 2 * r, 129 - 2 * r], [1, 700],
+                  [300, 1], [131, 275]):
+            T = 11 + k
+            u = rng.random([x + 2 * r for x in n]).astype(np.float32)
+            A = np.stack([u, u])
+            hosts.append((name, n, T, div, A))
+            items.append((name, n, T, torch.from_numpy(A.copy()).cuda(), None, div))
+    b = pyan5d.Batch(items, bt=bt)
+    b.run()
+    torch.cuda.synchronize()
+    for (name, n, T, div, A), it in zip(hosts, items):
+        ref = A.copy()
+        O.run(name, ref, n, T, divisor=div)
+        assert _same_bits(it[3][T % 2].cpu().numpy(), ref[T % 2]), (name, n, T, div)
+    b.close()
