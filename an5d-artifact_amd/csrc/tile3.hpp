@@ -9,13 +9,17 @@
 // computes the planes that still count (OP + 2*(BT-s)), so the overlap along
 // dim 0 costs loads but few operations.  Rows and columns give up BT cells on
 // every side that is not the grid's edge.
-// Bound by launch latency to 64^3, by vector issue above.  Measured by the
-// tuner, one step, best other kernel -> here: star3d1r 128^3 FP32 3.82 -> 2.69
-// us, FP64 5.83 -> 3.89; in FMA mode the boxes at every size whose steps are
-// bound by memory: j3d27pt FP32 512^3 287 -> 205 us, FP64 481 -> 412,
-// 257x300x411 134 -> 107.  The exact boxes stay with one step per launch (twice
-// the operations).  Eight planes a tile, one cell and four rows a lane: four
-// planes or two cells a lane were slower at every size but 64^3 (within 5 %).
+// Bound by launch latency to 64^3, by vector issue above.  One step, sweep ->
+// here: star3d1r 128^3 FP32 7.0 -> 5.6 us, FP64 12.7 -> 7.7; in FMA mode the boxes
+// where their steps are bound by memory: j3d27pt FP32 512^3 287 -> 205 us, FP64
+// 481 -> 412, 257x300x411 134 -> 107.  The exact boxes stay with one step per
+// launch (twice the operations).
+// Shapes (tile3_inst.hip): eight planes of 32 rows by 64 cells compute fewest
+// cells; where they are fewer than the CUs, four planes and 16 rows.  star3d1r
+// FP64 100x90x110, one step: 7.6 us on 104 tiles of eight planes, 5.3 on four
+// planes, 4.8 on four planes of 16 rows; 64^3 7.2, 4.9, 3.2; FP32 100x90x110 5.4,
+// 3.7, 3.5.  Tried: two cells a lane (slower from 128^3 on), four planes of two
+// rows on 16 waves (3-20 % slower than on 8).
 #pragma once
 
 #include "engine.hpp"

@@ -46,6 +46,10 @@ void add_tile3(std::vector<Variant>& out) {
 #define AN5D_CAT(a, b, c) AN5D_CAT2(a, b, c)
 void AN5D_CAT(register_tile3_, AN5D_SID, AN5D_F64)(std::vector<Variant>& out) {
   add_tile3<8, 1, 4, 8, BOX ? 3 : 4>(out);
+  if constexpr (!BOX) {
+    add_tile3<4, 1, 4, 8, 4>(out);
+    add_tile3<4, 1, 2, 8, 4>(out);
+  }
 }
 
 }  // namespace an5d

@@ -53,7 +53,7 @@ BENCH = [
 
 
 LADDER_2D = [256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192, 16384]
-LADDER_3D = [64, 128, 256, 512]
+LADDER_3D = [64, 96, 128, 192, 256, 512]
 
 
 def workloads(which):

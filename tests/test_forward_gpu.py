@@ -515,3 +515,22 @@ def test_register_tiles_division_modes(name, dt):
             pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=3, divisor=div)
             O.run(name, B, n, T, divisor=div)
             assert same(A[T % 2], B[T % 2])
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_3d_register_tiles_of_four_planes(dt):
+    """The tiles of four planes by 16 or 32 rows: exactly one tile, a plane, a
+    row or a cell more, at every depth; bit for bit the oracle."""
+    name = "star3d1r"
+    for v in pyan5d.variants(name, 0 if dt == np.float32 else 1):
+        if v["kind"] != 5:
+            continue
+        for bt in range(1, v["btmax"] + 1):
+            for n in ([4, 14, 62], [5, 14, 62], [4, 15, 62], [4, 30, 63], [13, 45, 127]):
+                T = bt + 1
+                print(f"case tiles {name} {np.dtype(dt).name} variant {v['index']} bt={bt} n={n}", flush=True)
+                A = rand_grid(name, n, dt, seed=sum(n) + bt)
+                B = A.copy()
+                pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt)
+                O.run(name, B, n, T)
+                assert same(A[T % 2], B[T % 2])
