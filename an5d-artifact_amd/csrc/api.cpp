@@ -186,6 +186,25 @@ int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long
   } else if (v.kind == kSweep && g.r <= 2) {
     body = g.r == 1 && bt * v.cj * v.ck <= 36 ? 6 : 2 * g.r + 1;
   }
+  // Grids past the 256 MB last-level cache wait for memory.  2D sweeps then want
+  // as many waves a SIMD as its registers hold (j2d5pt FP32 12000^2, one step: 73
+  // us at four, 76 at three, 83 at two; star2d4r FP64 6500^2 113 us at the one
+  // that fits, 146 at three), by an estimate that gives the compiled kernels'
+  // count: the rings and what the taps' rows take beside them.  And
+  // the LDS-staged planes of the 3D stars no more workgroups than run together,
+  // which share their halos in L2 (star3d4r FP32 400x420x390: 193 us with two a
+  // CU, 217 with three).
+  const bool past_llc = 2 * g.area * (v.dtype == kF64 ? 8 : 4) > (192LL << 20);
+  long long most_wgs = 1LL << 60;
+  if (past_llc && !tiles3 && v.kind == kSweep) {
+    const int w = v.dtype == kF64 ? 2 : 1;
+    const bool box = stencil_rt(v.stencil).ntaps > 4 * g.r + 1;
+    int regs = bt * (2 * g.r + 1) * v.ck * w + 28 + 5 * w * g.r + (w == 2 ? 4 : 0) + (box ? 5 * g.r * g.r * w : 0);
+    if (v.regcap > 0 && regs > v.regcap) regs = v.regcap;
+    lat = 512 / ((regs + 7) / 8 * 8);
+    lat = lat < 1 ? 1 : (lat > 5 ? 5 : lat);
+  }
+  if (past_llc && v.kind == kPlane && g.r > 1) most_wgs = 2 * cus;
   double best_t = 1e300;
   long long best = n0 < longest ? n0 : longest;
   // every count up to 64, then steps of a sixteenth
@@ -193,6 +212,7 @@ int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long
     const long long sl = cdiv(n0, nseg);
     const long long waves = cols && !tiles3 ? cdiv(ntk * nseg, 64) : ntk * nseg;
     const long long wgs = tiles3 ? ntk * ntj * nseg : cdiv(waves, v.nw);
+    if (wgs > most_wgs && nseg > cdiv(n0, longest)) break;
     const double share = (double)cdiv(wgs, cus) * v.nw / 4;
     const double planes = body > 1 ? (double)cdiv(sl + (long long)warm, body) * body : sl + warm;
     const double t = planes * (share > lat ? share : lat);
@@ -485,6 +505,50 @@ int default_bt(const StencilRT& s, int dtype) {
   return s.rad == 1 ? 2 : 1;
 }
 
+// Time per step of a 2D register-tile launch, in microseconds: a launch's own
+// time, and per step and for the loads and stores (3 steps) the tiles of the
+// busiest CU one after the other at the rate of the vector units.
+static double tile_step_us(const StencilRT& s, const Variant& v, int bt, const Geom& g, int mode, int cus) {
+  const long long TH = (long long)v.nw * v.cj, TW = 64LL * v.ck, H = (long long)bt * g.r;
+  if (TH <= 2 * H || TW <= 2 * H) return 1e300;
+  const long long nti = g.D0 > TH ? cdiv(g.D0 - 2 * H, TH - 2 * H) : 1;
+  const long long ntk = g.D2 > TW ? cdiv(g.D2 - 2 * H, TW - 2 * H) : 1;
+  const double ops = s.linear ? (mode == AN5D_FAST ? s.ntaps : s.fpp) : 2 * s.fpp;
+  const double tile_us = 4e-6 * (ops + 4) * (v.dtype == kF64 ? 2 : 1) * TH * TW;
+  return (2 + (bt + 3) * tile_us * cdiv(nti * ntk, cus)) / bt;
+}
+
+// A 2D register tile chosen by a table row of another size: which shape and
+// depth fit depends on how many tiles of them the busiest CU gets, so the row
+// stands only if no other is 10 % faster by the estimate above.  Its constants
+// were fitted to every shape and depth on 14 grids (245x315 .. 2273x2923, six of
+// them 4:1) of five stencils in both dtypes and FMA mode: the rows alone are 8.7
+// % off the best in the geometric mean (74 % at 1000x3001), with the rule 2.5 %;
+// without the 10 % 2.2 %, but more grids get slower.
+static void fit_tile(const an5d_problem* p, int mode, const std::vector<const Variant*>& vs, const Variant** v,
+                     int* bt) {
+  Geom g;
+  std::string err;
+  if (!make_geom(p, g, err) || g.dim != 2) return;
+  // larger grids are bound by memory, which the estimate leaves out (j2d5pt FP32
+  // 2600x10400: 23.5 us at its choice, 20.0 on streams)
+  if (2 * g.area * (p->dtype == AN5D_FLOAT64 ? 8 : 4) > (128LL << 20)) return;
+  const StencilRT& s = stencil_rt(p->stencil);
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  double best = 0.9 * tile_step_us(s, **v, *bt, g, mode, cus);
+  for (const Variant* x : vs) {
+    if (x->kind != kTile) continue;
+    for (int k = 1; k <= x->btmax; k++) {
+      const double t = tile_step_us(s, *x, k, g, mode, cus);
+      if (t < best) {
+        best = t;
+        *v = x;
+        *bt = k;
+      }
+    }
+  }
+}
+
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,
             int* slout) {
   const auto& vs = variants_of(p->stencil, p->dtype);
@@ -504,7 +568,10 @@ int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout,
     if (tuned_lookup(p, mode, &tc) && tc.variant < (int)vs.size() &&
         (want_bt == 0 || want_bt <= vs[tc.variant]->btmax)) {
       v = vs[tc.variant];
-      if (want_bt == 0) want_bt = tc.bt;
+      if (want_bt == 0) {
+        want_bt = tc.bt;
+        if (!tc.same_size && v->kind == kTile) fit_tile(p, mode, vs, &v, &want_bt);
+      }
       if (sl == 0) sl = tc.sl;
     } else {
       v = vs[0];  // first sweep shape, or the direct kernel when none exists

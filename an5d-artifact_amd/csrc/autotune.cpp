@@ -188,7 +188,8 @@ bool tuned_lookup(const an5d_problem* p, int mode, TunedChoice* out) {
   if (!best || best_d > log(8.0)) return false;  // only reuse within 8x of the size
   out->variant = best->variant;
   out->bt = best->bt;
-  out->sl = (best->n[0] == p->n[0] && best->n[1] == p->n[1] && best->n[2] == p->n[2]) ? best->sl : 0;
+  out->same_size = best->n[0] == p->n[0] && best->n[1] == p->n[1] && best->n[2] == p->n[2];
+  out->sl = out->same_size ? best->sl : 0;
   return true;
 }
 

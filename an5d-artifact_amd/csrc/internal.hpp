@@ -32,6 +32,7 @@ struct LaunchPlan {
 
 struct TunedChoice {
   int variant, bt, sl;
+  bool same_size;  // the row was measured at this problem's extents
 };
 
 int fail(int code, const std::string& msg);

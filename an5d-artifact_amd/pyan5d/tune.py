@@ -54,6 +54,8 @@ BENCH = [
 
 LADDER_2D = [256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096, 6144, 8192, 16384]
 LADDER_3D = [64, 96, 128, 192, 256, 512]
+# the radius-1 boxes change kernel between 256^3 and 512^3; the stars do not
+LADDER_BOX3D1 = {np.float32: [320, 400], np.float64: [320]}
 
 
 def workloads(which):
@@ -61,8 +63,9 @@ def workloads(which):
     if which in ("ladder", "all"):
         seen = {(s, np.dtype(d).name, tuple(n), m) for s, d, n, ms, _ in out for m in ms}
         for s in STENCILS_2D + STENCILS_3D:
-            for n in [[x] * 2 for x in LADDER_2D] if s in STENCILS_2D else [[x] * 3 for x in LADDER_3D]:
-                for dt in (np.float32, np.float64):
+            for dt in (np.float32, np.float64):
+                sides = LADDER_3D + (LADDER_BOX3D1[dt] if s in ("box3d1r", "j3d27pt") else [])
+                for n in [[x] * 2 for x in LADDER_2D] if s in STENCILS_2D else [[x] * 3 for x in sides]:
                     modes = tuple(m for m in (EXACT, FAST) if (s, np.dtype(dt).name, tuple(n), m) not in seen)
                     if modes:
                         out.append((s, dt, n, modes, 100))

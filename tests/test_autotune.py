@@ -33,6 +33,32 @@ def test_tune_table_roundtrip(tmp_path):
     pyan5d.tune_clear()
 
 
+def test_tile_choice_for_sizes_between_the_rows(tmp_path):
+    """A row that names a register tile: at its own size it stands; at another
+    size the choice is a register tile whose depth its shape holds; a caller's
+    depth or variant stands."""
+    path = tmp_path / "t.tsv"
+    for dt, f in ((pyan5d.FLOAT32, np.float32), (pyan5d.FLOAT64, np.float64)):
+        for name in ("j2d5pt", "star2d2r", "star2d4r", "box2d2r", "gradient2d"):
+            vs = pyan5d.variants(name, dt)
+            tiles = [v for v in vs if v["kind"] == 5]
+            row = tiles[-1]
+            path.write_text(f"{name} {dt} 0 1024 1024 0 {row['index']} 2 0 1.0\n")
+            pyan5d.tune_clear()
+            pyan5d.tune_load(str(path))
+            at = pyan5d.resolve_config(name, [1024, 1024], f)
+            assert (at["variant"], at["bt"]) == (row["index"], 2)
+            for n in ([1, 400000], [400000, 1], [800, 800], [1000, 3001], [3001, 1000], [400, 1300]):
+                c = pyan5d.resolve_config(name, n, f)
+                v = vs[c["variant"]]
+                assert v["kind"] == 5 and 1 <= c["bt"] <= v["btmax"], (name, n, c)
+                c = pyan5d.resolve_config(name, n, f, bt=1)
+                assert (c["variant"], c["bt"]) == (row["index"], 1)
+                c = pyan5d.resolve_config(name, n, f, variant=tiles[0]["index"], bt=2)
+                assert (c["variant"], c["bt"]) == (tiles[0]["index"], 2)
+    pyan5d.tune_clear()
+
+
 def test_tune_table_records_register_cap(tmp_path):
     """The cap column: a capped twin's deep block reports its cap, its
     shallow blocks (which share the uncapped kernels) report none."""

@@ -534,3 +534,18 @@ def test_3d_register_tiles_of_four_planes(dt):
                 pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt)
                 O.run(name, B, n, T)
                 assert same(A[T % 2], B[T % 2])
+
+
+@pytest.mark.parametrize("name", ["j2d5pt", "j2d9pt-gol", "star2d2r", "star2d4r", "box2d2r", "gradient2d"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_default_choice_on_ragged_grids(name, dt):
+    """The kernel and depth that a call without a configuration takes, at sizes
+    between the table's rows: long, tall and odd grids; bit for bit the oracle."""
+    for n in ([3, 9001], [9001, 3], [311, 517], [256, 1025], [700, 901]):
+        T = 18
+        print(f"case default {name} {np.dtype(dt).name} n={n}", flush=True)
+        A = rand_grid(name, n, dt, seed=sum(n))
+        B = A.copy()
+        pyan5d.forward_host(name, A, n, T)
+        O.run(name, B, n, T)
+        assert same(A[T % 2], B[T % 2])
