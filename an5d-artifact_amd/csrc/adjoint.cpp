@@ -128,6 +128,14 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
     bt_pref = bt;
     sl_pref = 0;
   }
+  // the block's few steps on a large FP32 grid are faster on the sweep than on a
+  // tile chosen for its depth (j2d9pt 3700x3900, 24 steps: 1145 -> 1001 us)
+  if ((!cfg || cfg->variant < 0) && ap.fwd->kind == kTile && p->dtype == AN5D_FLOAT32 &&
+      2 * ap.g.area * 4 > (48LL << 20) && vs[0]->kind == kSweep && vs[0]->btmax >= ap.adj->btmax && vs[0]->btmax >= bt) {
+    fc.variant = 0;
+    rc = resolve(p, &fc, &ap.fwd, &bt_pref, &sl_pref);
+    if (rc) return rc;
+  }
   if (bt > ap.adj->btmax || bt > ap.fwd->btmax) {
     if (cfg && cfg->bt > 0) return fail(AN5D_E_UNSUPPORTED, "bt exceeds the adjoint or forward btmax");
     bt = ap.adj->btmax < ap.fwd->btmax ? ap.adj->btmax : ap.fwd->btmax;
@@ -263,12 +271,16 @@ static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, d
     if (sl < kMinSlLean) sl = kMinSlLean;
     if (sl > n0) sl = n0;
   } else if (ap.sl <= 0) {
+    // kernels that hold one wave a SIMD (the wide boxes) gain nothing from a
+    // second (box2d3r 2800x2500, 24 steps: 12.1 ms on one round, 14.4 on two)
+    const int occ = !slots && ap.adj->occupancy ? ap.adj->occupancy(k) * (int)nw / 4 : 2;
+    const double least = occ == 1 ? 1.0 : 2.0;
     for (long long nseg = 1; nseg <= n0; nseg++) {
       const long long s = cdiv(n0, nseg);
       if (s < minsl && nseg > 1) break;
       const double share = ceil((double)cdiv(ntk * nseg, nw) / cus) * nw / 4;
       const double planes = (double)cdiv(s + HU + DLT + k * R, ring - 1) * (ring - 1);
-      const double t = planes * ck * (share > 2.0 ? share : 2.0);
+      const double t = planes * ck * (share > least ? share : least);
       if (t < t_best) {
         t_best = t;
         sl = s;
