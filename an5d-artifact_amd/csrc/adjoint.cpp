@@ -129,8 +129,10 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
     sl_pref = 0;
   }
   // the block's few steps on a large FP32 grid are faster on the sweep than on a
-  // tile chosen for its depth (j2d9pt 3700x3900, 24 steps: 1145 -> 1001 us)
-  if ((!cfg || cfg->variant < 0) && ap.fwd->kind == kTile && p->dtype == AN5D_FLOAT32 &&
+  // tile chosen for its depth (j2d9pt 3700x3900, 24 steps: 1145 -> 1001 us); not
+  // with a division (over 118, 4096^2, 64 steps: 3073 us on the tile, 3267)
+  const double divisor = p->divisor < 0 ? stencil_rt(p->stencil).divisor : p->divisor;
+  if (divisor == 0 && (!cfg || cfg->variant < 0) && ap.fwd->kind == kTile && p->dtype == AN5D_FLOAT32 &&
       2 * ap.g.area * 4 > (48LL << 20) && vs[0]->kind == kSweep && vs[0]->btmax >= ap.adj->btmax && vs[0]->btmax >= bt) {
     fc.variant = 0;
     rc = resolve(p, &fc, &ap.fwd, &bt_pref, &sl_pref);
