@@ -826,11 +826,16 @@ extern "C" int an5d_forward_host(const an5d_problem* p, void* A, const an5d_conf
   char* h1 = h0 + gb;
   char* d0 = static_cast<char*>(dA);
   char* d1 = d0 + gb;
+  // The array may be pinned memory that work already enqueued on the device still
+  // writes or reads (a copy on the null stream, say): the threads that copy it
+  // below are ordered after no stream, so wait for all of them.
+  hipError_t e = hipDeviceSynchronize();
+  if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
   // The first launch writes the whole interior of buffer 1: of that buffer only
   // the halo is read, so only the halo goes up.
   rc = staging_upload(*ring, d0, h0, gb);
   if (rc == AN5D_OK) rc = staging_upload_halo(*ring, d1, h1, g, esz);
-  hipError_t e = hipStreamSynchronize(ring->st);
+  e = hipStreamSynchronize(ring->st);
   if (rc) return rc;
   if (e != hipSuccess) return hip_fail(e, "H2D copies");
   int launches = 0;

@@ -335,6 +335,36 @@ def test_forward_host_from_several_threads():
         assert np.array_equal(o[T % 2], ref[T % 2])
 
 
+def test_forward_host_waits_for_copies_under_way(torch_cuda):
+    """A pinned host array that a copy enqueued on the null stream is still to
+    fill (behind a few milliseconds of work): the call waits for it; and a copy
+    out of the array enqueued before the call takes the state before it."""
+    torch = torch_cuda
+    name, n, T = "j2d5pt", [500, 700], 6
+    print("case host array with copies under way", name, flush=True)
+    A = rand_grid(name, n, np.float32, seed=3)
+    ref = A.copy()
+    O.run(name, ref, n, T)
+    dev = torch.from_numpy(A).cuda()
+    pinned = torch.zeros(A.shape, pin_memory=True)
+    back = torch.zeros_like(dev)
+    m = torch.rand(4096, 4096, device="cuda")
+    torch.mm(m, m)
+    torch.cuda.synchronize()
+    for _ in range(40):
+        torch.mm(m, m)
+    pinned.copy_(dev, non_blocking=True)
+    pyan5d.forward_host(name, pinned.numpy(), n, T)
+    assert same(pinned.numpy()[T % 2], ref[T % 2])
+    pinned.copy_(torch.from_numpy(A))
+    for _ in range(40):
+        torch.mm(m, m)
+    back.copy_(pinned, non_blocking=True)
+    pyan5d.forward_host(name, pinned.numpy(), n, T)
+    torch.cuda.synchronize()
+    assert same(back.cpu().numpy(), A)
+
+
 @pytest.mark.parametrize("name", ["box3d2r", "box3d3r", "box3d4r"])
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 def test_box3d_column_kernel_ragged_grids(name, dt):
