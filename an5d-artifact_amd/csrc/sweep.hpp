@@ -867,7 +867,11 @@ __device__ __forceinline__ void sweep_body(const SweepArgs<T>& a, int tile = -1)
           ring[S][P - 1] = out;
         } else {
           if constexpr (NBWAIT) {
-            if (lane == 0) __hip_atomic_store(ready + w, n + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            // every lane's rows, written and read, come before the count: the
+            // fence is the whole wave's, the store is lane 0's
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            if (lane == 0) __hip_atomic_store(ready + w, n + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           }
           if (n >= 2 * BT * R && n < nit) store_plane(out, p_in - BT * R, a.dst);
         }

@@ -579,3 +579,24 @@ def test_default_choice_on_ragged_grids(name, dt):
         pyan5d.forward_host(name, A, n, T)
         O.run(name, B, n, T)
         assert same(A[T % 2], B[T % 2])
+
+
+def test_star3d_neighbour_waits():
+    """FP32 exact star3d1r at three steps a launch and more, where the waves wait
+    for their two neighbours: ragged grids of several workgroups and segments, the
+    general and the shared-product form; bit for bit the oracle, twice."""
+    name = "star3d1r"
+    for v in pyan5d.variants(name, 0):
+        if v["kind"] != 0:
+            continue
+        for bt in range(3, v["btmax"] + 1):
+            for n, sl in (([1, 1, 1], 0), ([29, 70, 131], 7), ([61, 33, 200], 0)):
+                print(f"case neighbour waits variant {v['index']} bt={bt} n={n} sl={sl}", flush=True)
+                A = rand_grid(name, n, np.float32, seed=sum(n) + bt)
+                ref = A.copy()
+                O.run(name, ref, n, bt + 1)
+                for mode in (pyan5d.EXACT, pyan5d.EXACT_GENERAL):
+                    for _ in range(2):
+                        B = A.copy()
+                        pyan5d.forward_host(name, B, n, bt + 1, variant=v["index"], bt=bt, sl=sl, mode=mode)
+                        assert same(B[(bt + 1) % 2], ref[(bt + 1) % 2])
