@@ -163,10 +163,11 @@ int device_cus() {
 // the 2*bt*R warm-up planes of the sweeps and what fills whole loop bodies.
 // L and the warm-up were fitted to the times of every segment length 1 .. 128
 // over 256^2 .. 8192^2 and 64^3 .. 384^3 (squares, cubes and ragged
-// rectangles, both dtypes): the choice is 1-3 % off the best in the geometric
-// mean, where "as many segments as fill the resident workgroups in one round,
-// 8*bt*R planes at least" was 1.5-2.1 times off (a 256^2 grid got 16 waves).
-int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long ntj) {
+// rectangles, both dtypes).  Against "as many segments as fill the resident
+// workgroups in one round, 8*bt*R planes at least": 0.63 of the time in the
+// geometric mean over 5280 calls of every 2D sweep, depth and mode at 700^2 ..
+// 5000^2 (a 256^2 grid got 16 waves), 6 % of them 3 % or more slower.
+int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long ntj, int mode) {
   const long long n0 = g.D0 - 2 * g.r;
   const long long cus = device_cus() > 0 ? device_cus() : 256;
   const bool tiles3 = g.dim == 3;     // a segment holds ntk * ntj workgroups, else ntk waves
@@ -186,16 +187,25 @@ int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long
   } else if (v.kind == kSweep && g.r <= 2) {
     body = g.r == 1 && bt * v.cj * v.ck <= 36 ? 6 : 2 * g.r + 1;
   }
-  // Grids past the 256 MB last-level cache wait for memory.  2D sweeps then want
-  // as many waves a SIMD as its registers hold (j2d5pt FP32 12000^2, one step: 73
-  // us at four, 76 at three, 83 at two; star2d4r FP64 6500^2 113 us at the one
-  // that fits, 146 at three), by an estimate that gives the compiled kernels'
-  // count: the rings and what the taps' rows take beside them.  And
-  // the LDS-staged planes of the 3D stars no more workgroups than run together,
-  // which share their halos in L2 (star3d4r FP32 400x420x390: 193 us with two a
-  // CU, 217 with three).
+  // Grids past the 256 MB last-level cache wait for memory: 2D sweeps want as
+  // many waves a SIMD as their registers hold.  Where one round of them has
+  // segments of 8*bt*R planes, that round is the choice (the model: 1.02 of its
+  // time in the geometric mean over 5600 calls at 4000^2 .. 12000^2, up to 1.43;
+  // box2d3r FP64 FMA 12000^2, two steps a launch: 471 us a step in one round,
+  // 573 at half its waves).  Where it has not, the model with L from an estimate
+  // of the registers: 0.934 of the round's time at that least length over 1561
+  // calls, and 0.935 with the compiler's count, capped at 5, in its place.
+  // And the LDS-staged planes of the 3D stars want no more workgroups than run
+  // together, which share their halos in L2 (star3d4r FP32 400x420x390: 193 us
+  // with two a CU, 217 with three).
   const bool past_llc = 2 * g.area * (v.dtype == kF64 ? 8 : 4) > (192LL << 20);
   long long most_wgs = 1LL << 60;
+  const int occ = v.occ[bt] ? v.occ[bt](mode) : 0;  // workgroups a CU holds (0: not a 2D sweep, or no device)
+  if (past_llc && occ > 0) {
+    const long long nseg = occ * cus * v.nw / ntk;
+    const long long round = cdiv(n0, nseg > 1 ? nseg : 1);
+    if (round >= 8LL * bt * g.r) return (int)round;
+  }
   if (past_llc && !tiles3 && v.kind == kSweep) {
     const int w = v.dtype == kF64 ? 2 : 1;
     const bool box = stencil_rt(v.stencil).ntaps > 4 * g.r + 1;
@@ -204,6 +214,9 @@ int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long
     lat = 512 / ((regs + 7) / 8 * 8);
     lat = lat < 1 ? 1 : (lat > 5 ? 5 : lat);
   }
+  // a kernel that holds one wave a SIMD gains nothing from a second (box2d4r FP32
+  // 5000^2, three steps: 187 us a step in one round, 222 in two)
+  if (occ > 0 && occ * v.nw <= 4) lat = 1;
   if (past_llc && v.kind == kPlane && g.r > 1) most_wgs = 2 * cus;
   double best_t = 1e300;
   long long best = n0 < longest ? n0 : longest;
@@ -250,7 +263,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     if (g.dim == 2) {
       // lanes of ck cells over the segments, row-major
       const long long ntk = cdiv(nk, v.ck);
-      if (sl <= 0) sl = default_sl(v, bt, g, ntk, 1);
+      if (sl <= 0) sl = default_sl(v, bt, g, ntk, 1, mode);
       if (sl > n0) sl = (int)n0;
       const long long nseg = cdiv(n0, sl);
       if (ntk * nseg >= (1LL << 30)) { err = "grid too large"; return false; }
@@ -263,7 +276,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     // lanes of ck cells over the plane, row-major, in blocks of 256 per segment
     const long long ntk = cdiv(nk, v.ck), nblk = cdiv(ntk * nj, 256);
     if (ntk * nj >= (1LL << 30)) { err = "grid too large"; return false; }
-    if (sl <= 0) sl = default_sl(v, bt, g, nblk, 1);
+    if (sl <= 0) sl = default_sl(v, bt, g, nblk, 1, mode);
     const long long nseg = cdiv(n0, sl);
     a.ntk = (int)ntk; a.ntj = (int)nblk; a.nseg = (int)nseg; a.sl = sl;
     a.SK = v.ck; a.SJ = 1;
@@ -302,7 +315,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     if (g.dim != 3) { err = "the plane kernel is 3D only"; return false; }
     const long long TK = 64LL * v.ck, TJ = (long long)v.nw * v.cj;
     const long long ntk = cdiv(nk, TK), ntj = cdiv(nj, TJ);
-    if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj);
+    if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj, mode);
     const long long nseg = cdiv(n0, sl);
     a.ntk = (int)ntk; a.ntj = (int)ntj; a.nseg = (int)nseg; a.sl = sl;
     a.SK = (int)TK; a.SJ = (int)TJ;
@@ -329,7 +342,7 @@ bool plan_launch(const Variant& v, int bt, const Geom& g, int sl, LaunchPlan& lp
     if (SJ <= 0) { err = "bt too deep for this variant's tile height"; return false; }
     ntj = cdiv(nj, SJ);
   }
-  if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj);
+  if (sl <= 0) sl = default_sl(v, bt, g, ntk, ntj, mode);
   const long long nseg = cdiv(n0, sl);
   a.ntk = (int)ntk; a.ntj = (int)ntj; a.nseg = (int)nseg; a.sl = sl;
   a.SK = (int)SK; a.SJ = (int)SJ;

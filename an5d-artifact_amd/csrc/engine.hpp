@@ -75,6 +75,8 @@ struct Variant {
   // private (scratch) bytes per thread of fn_share[bt] (-1 unknown): a kernel
   // that spills is slower than the general form and is not used
   int (*share_scratch[kMaxBT + 1])();
+  // 2D sweeps: resident workgroups per CU of fn[bt] (mode 0), fn_fast[bt] (1), fn_share[bt] (2)
+  int (*occ[kMaxBT + 1])(int mode);
   LaunchFn fn_mid[kMaxBT + 1];  // exact mode storing intermediate stages (2D, bt <= kMaxMidBT)
 };
 

@@ -54,6 +54,27 @@ int share_scratch_once() {
   return n;
 }
 
+// Resident workgroups per CU of a 2D sweep (0 if the query fails); computed once,
+// on the first device that asks (every device is a gfx950 with the same resources).
+template <int BT, int CK, int CJ, int NW, bool EXACT, bool SHARE, int WPE>
+int occupancy_once() {
+  static_assert(sweep_lds_bytes<SID, T, CK, CJ, NW>(BT) == 0, "2D waves share no LDS");
+  static const int n = [] {
+    const void* k = reinterpret_cast<const void*>(sweep_fn<BT, CK, CJ, NW, EXACT, false, SHARE, WPE>());
+    int blocks = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 64 * NW, 0) != hipSuccess) return 0;
+    return blocks;
+  }();
+  return n;
+}
+template <int BT, int CK, int CJ, int NW, int WPE>
+int occupancy_sweep(int mode) {
+  if constexpr (kShare && WPE == 0)
+    if (mode == 2) return occupancy_once<BT, CK, CJ, NW, true, true, 0>();
+  return mode == 1 ? occupancy_once<BT, CK, CJ, NW, false, false, WPE>()
+                   : occupancy_once<BT, CK, CJ, NW, true, false, WPE>();
+}
+
 template <int CK, bool EXACT>
 hipError_t launch_direct(const LaunchArgs& a, dim3 grid, dim3 block, size_t lds, hipStream_t st) {
   hipLaunchKernelGGL((direct_kernel<SID, T, CK, EXACT>), grid, block, lds, st, to_args<T>(a));
@@ -155,6 +176,7 @@ void add_sweep(std::vector<Variant>& out) {
         v.fn_share[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, false, true>;
         v.share_scratch[BT] = &share_scratch_once<BT, sh.ck, sh.cj, sh.nw>;
       }
+      if constexpr (Def<SID>::dim == 2) v.occ[BT] = &occupancy_sweep<BT, sh.ck, sh.cj, sh.nw, 0>;
       // intermediate-stage outputs: the adjoint's checkpointing forward pass (2D, exact)
       if constexpr (Def<SID>::dim == 2 && BT >= 2 && BT <= kMaxMidBT)
         v.fn_mid[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, true>;
@@ -187,6 +209,7 @@ void add_capped(std::vector<Variant>& out) {
       v.lds[BT] = sweep_lds_bytes<SID, T, sh.ck, sh.cj, sh.nw>(BT);
       v.fn[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, false, false, C>;
       v.fn_fast[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, false, false, false, C>;
+      if constexpr (Def<SID>::dim == 2) v.occ[BT] = &occupancy_sweep<BT, sh.ck, sh.cj, sh.nw, C>;
       if constexpr (Def<SID>::dim == 2 && BT >= 2 && BT <= kMaxMidBT)
         v.fn_mid[BT] = &launch_sweep<BT, sh.ck, sh.cj, sh.nw, true, true>;
     });

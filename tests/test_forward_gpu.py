@@ -600,3 +600,20 @@ def test_star3d_neighbour_waits():
                         B = A.copy()
                         pyan5d.forward_host(name, B, n, bt + 1, variant=v["index"], bt=bt, sl=sl, mode=mode)
                         assert same(B[(bt + 1) % 2], ref[(bt + 1) % 2])
+
+
+@pytest.mark.parametrize("name,dt,mode,bt,n,ck,waves", [
+    ("box2d3r", np.float64, pyan5d.FAST, 2, [12000, 12000], 4, 2),
+    ("box2d3r", np.float64, pyan5d.FAST, 2, [14000, 3500], 4, 2),
+    ("box2d4r", np.float32, pyan5d.EXACT, 3, [5000, 5000], 4, 1)])
+def test_segments_of_large_grids_fill_one_round(name, dt, mode, bt, n, ck, waves):
+    """The default segment length of a 2D sweep on a grid that fills the chip: as
+    many waves as the kernel's registers hold (the last argument, per SIMD), no
+    second round and not half of one."""
+    r = O.info(name)["rad"]
+    print(f"case segments {name} {np.dtype(dt).name} n={n}", flush=True)
+    v = pyan5d.variants(name, 0 if dt == np.float32 else 1)[0]
+    assert v["kind"] == 0 and v["ck"] == ck
+    sl = pyan5d.resolve_config(name, n, dt, mode=mode, bt=bt, variant=0)["sl"]
+    runs = -(-n[0] // sl) * -(-n[1] // (64 * ck - 2 * bt * r))
+    assert 0.9 * waves * 1024 <= runs <= waves * 1024
