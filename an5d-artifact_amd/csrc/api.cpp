@@ -192,9 +192,10 @@ int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long
   // segments of 8*bt*R planes, that round is the choice (the model: 1.02 of its
   // time in the geometric mean over 5600 calls at 4000^2 .. 12000^2, up to 1.43;
   // box2d3r FP64 FMA 12000^2, two steps a launch: 471 us a step in one round,
-  // 573 at half its waves).  Where it has not, the model with L from an estimate
-  // of the registers: 0.934 of the round's time at that least length over 1561
-  // calls, and 0.935 with the compiler's count, capped at 5, in its place.
+  // 573 at half its waves), and that length where it has a tenth less (435
+  // calls: 0.99 of the model's time; a fifth less, 356 calls: 1.06).  Else the
+  // model with L from an estimate of the registers (0.93 of the time of that
+  // least length over 1561 calls; the compiler's count in its place, 0.935).
   // And the LDS-staged planes of the 3D stars want no more workgroups than run
   // together, which share their halos in L2 (star3d4r FP32 400x420x390: 193 us
   // with two a CU, 217 with three).
@@ -204,7 +205,8 @@ int default_sl(const Variant& v, int bt, const Geom& g, long long ntk, long long
   if (past_llc && occ > 0) {
     const long long nseg = occ * cus * v.nw / ntk;
     const long long round = cdiv(n0, nseg > 1 ? nseg : 1);
-    if (round >= 8LL * bt * g.r) return (int)round;
+    const long long least = 8LL * bt * g.r < n0 ? 8LL * bt * g.r : n0;
+    if (10 * round >= 9 * least) return (int)(round > least ? round : least);
   }
   if (past_llc && !tiles3 && v.kind == kSweep) {
     const int w = v.dtype == kF64 ? 2 : 1;
