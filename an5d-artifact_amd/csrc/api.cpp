@@ -564,6 +564,32 @@ static void fit_tile(const an5d_problem* p, int mode, const std::vector<const Va
   }
 }
 
+// A caller's depth beyond the one that a table row was measured at.  A kernel
+// held to fewer registers spills there: its uncapped twin (star2d3r FP64
+// 3500x3500, six steps: 9.8 times faster, star2d4r FP64 FMA, four: 5.4 times).  A
+// 2D register tile that gives up too much of itself: the stencil's sweep.  Of
+// the tiles that keep less than 0.3 more than half are slower than it, up to 1.8
+// times; between 0.3 and 0.5 so are those past 128 MB (1.07 of its time in the
+// geometric mean of 20 calls; star2d2r FP64 5000^2, eight steps, 1.23), those
+// below take 0.71 of it.
+static const Variant* deeper_variant(const an5d_problem* p, const std::vector<const Variant*>& vs, const Variant* v,
+                                     int bt) {
+  Geom g;
+  std::string err;
+  if (!make_geom(p, g, err)) return v;
+  if (v->kind == kSweep && v->regcap > 0) {
+    for (const Variant* x : vs)
+      if (x->kind == kSweep && x->regcap == 0 && x->ck == v->ck && x->cj == v->cj && x->nw == v->nw) return x;
+  }
+  if (v->kind == kTile && g.dim == 2 && vs[0]->kind == kSweep && vs[0]->btmax >= bt) {
+    const double TH = (double)v->nw * v->cj, TW = 64.0 * v->ck, H = (double)bt * g.r;
+    const double kept = TH > 2 * H && TW > 2 * H ? (1 - 2 * H / TH) * (1 - 2 * H / TW) : 0;
+    const bool large = 2 * g.area * (p->dtype == AN5D_FLOAT64 ? 8 : 4) > (128LL << 20);
+    if (kept < (large ? 0.5 : 0.3)) return vs[0];
+  }
+  return v;
+}
+
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,
             int* slout) {
   const auto& vs = variants_of(p->stencil, p->dtype);
@@ -586,8 +612,10 @@ int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout,
       if (want_bt == 0) {
         want_bt = tc.bt;
         if (!tc.same_size && v->kind == kTile) fit_tile(p, mode, vs, &v, &want_bt);
+      } else if (want_bt > tc.bt) {
+        v = deeper_variant(p, vs, v, want_bt);
       }
-      if (sl == 0) sl = tc.sl;
+      if (sl == 0 && v == vs[tc.variant]) sl = tc.sl;
     } else {
       v = vs[0];  // first sweep shape, or the direct kernel when none exists
     }

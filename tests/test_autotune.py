@@ -59,6 +59,38 @@ def test_tile_choice_for_sizes_between_the_rows(tmp_path):
     pyan5d.tune_clear()
 
 
+def test_callers_depth_beyond_the_rows(tmp_path):
+    """A caller's depth beyond the row's: the uncapped twin of a register-capped
+    sweep, the sweep instead of a 2D register tile that keeps too little of
+    itself; at the row's depth and below it the row's kernel stands."""
+    path = tmp_path / "t.tsv"
+
+    def load(name, dt, n, v, bt):
+        path.write_text(f"{name} {dt} 0 {n} {n} 0 {v} {bt} 0 1.0\n")
+        pyan5d.tune_clear()
+        pyan5d.tune_load(str(path))
+
+    for name, dt, f, row_bt, deep in (("star2d3r", 1, np.float64, 3, 6), ("star2d4r", 1, np.float64, 2, 4),
+                                      ("j2d9pt", 0, np.float32, 5, 8)):
+        vs = pyan5d.variants(name, dt)
+        v = [v for v in vs if v["kind"] == 0 and v["regcap"] > 0][0]
+        load(name, dt, 8192, v["index"], row_bt)
+        for n in ([8192, 8192], [3500, 3500]):
+            assert pyan5d.resolve_config(name, n, f, bt=row_bt)["variant"] == v["index"]
+            assert pyan5d.resolve_config(name, n, f, bt=1)["variant"] == v["index"]
+            c = vs[pyan5d.resolve_config(name, n, f, bt=deep)["variant"]]
+            assert c["kind"] == 0 and c["regcap"] == 0
+            assert [c[k] for k in ("ck", "cj", "nw")] == [v[k] for k in ("ck", "cj", "nw")]
+    for name, dt, f, deep in (("star2d2r", 1, np.float64, 8), ("star2d3r", 0, np.float32, 4)):
+        vs = pyan5d.variants(name, dt)
+        v = [v for v in vs if v["kind"] == 5 and v["btmax"] >= deep][0]
+        load(name, dt, 4096, v["index"], 2)
+        for n in ([4096, 4096], [7000, 7000]):
+            assert pyan5d.resolve_config(name, n, f, bt=2)["variant"] == v["index"]
+            assert vs[pyan5d.resolve_config(name, n, f, bt=deep)["variant"]]["kind"] == 0
+    pyan5d.tune_clear()
+
+
 def test_tune_table_records_register_cap(tmp_path):
     """The cap column: a capped twin's deep block reports its cap, its
     shallow blocks (which share the uncapped kernels) report none."""
