@@ -273,21 +273,38 @@ static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, d
     if (sl < kMinSlLean) sl = kMinSlLean;
     if (sl > n0) sl = n0;
   } else if (ap.sl <= 0) {
-    // kernels that hold one wave a SIMD (the wide boxes) gain nothing from a
-    // second (box2d3r 2800x2500, 24 steps: 12.1 ms on one round, 14.4 on two)
-    const int occ = !slots && ap.adj->occupancy ? ap.adj->occupancy(k) * (int)nw / 4 : 2;
-    const double least = occ == 1 ? 1.0 : 2.0;
-    for (long long nseg = 1; nseg <= n0; nseg++) {
-      const long long s = cdiv(n0, nseg);
-      if (s < minsl && nseg > 1) break;
-      const double share = ceil((double)cdiv(ntk * nseg, nw) / cus) * nw / 4;
+    // waves a SIMD holds; one that holds one (radius 1 with 5 taps, the wide boxes
+    // and stars) gains nothing from a second (box2d3r 2800x2500, 24 steps: 12.1 ms
+    // on one round, 14.4 on two)
+    const int held = !slots && ap.adj->occupancy ? ap.adj->occupancy(k) * (int)nw / 4 : 2;
+    const double least = held == 1 ? 1.0 : 2.0;
+    auto share_of = [&](long long nseg) { return ceil((double)cdiv(ntk * nseg, nw) / cus) * nw / 4; };
+    auto time = [&](long long s, long long nseg) {
+      const double share = share_of(nseg);
       const double planes = (double)cdiv(s + HU + DLT + k * R, ring - 1) * (ring - 1);
-      const double t = planes * ck * (share > least ? share : least);
-      if (t < t_best) {
-        t_best = t;
-        sl = s;
+      return planes * ck * (share > least ? share : least);
+    };
+    // and loses by every SIMD left idle, which whole ring lengths hide from the
+    // model: one round where its segments have 16 planes (24 steps, model -> round:
+    // star2d4r 3700x3900 4241 -> 3854 us, box2d3r 2800x2500 12.3 -> 10.9 ms, box2d4r
+    // 4000x1000 30.4 -> 25.6 ms, star2d1r 2000^2 500 -> 454 us; the worst of 77,
+    // star2d4r 1000x4000, 1373 -> 1418)
+    const long long most = held == 1 ? (long long)(4 * cus) / ntk : 0;
+    const long long round = cdiv(n0, most > 1 ? most : 1);
+    if (held == 1 && round >= kMinSlLean) {
+      sl = round;
+      t_best = time(sl, cdiv(n0, sl));
+    } else {
+      for (long long nseg = 1; nseg <= n0; nseg++) {
+        const long long s = cdiv(n0, nseg);
+        if (s < minsl && nseg > 1) break;
+        const double t = time(s, nseg);
+        if (t < t_best) {
+          t_best = t;
+          sl = s;
+        }
+        if (share_of(nseg) > 12) break;
       }
-      if (share > 12) break;
     }
   }
   l.D0 = (int)ap.g.D0;
@@ -348,6 +365,29 @@ extern "C" int an5d_adjoint_workspace(const an5d_problem* p, const an5d_config* 
                                   " padded grids: one per bt-step block) exceeds the device's " +
                                   std::to_string(total_b >> 20) + " MiB; use a larger bt or fewer steps");
   (void)hipGetLastError();
+  return AN5D_OK;
+}
+
+extern "C" int an5d_adjoint_resolve(const an5d_problem* p, const an5d_config* cfg, an5d_adjoint_choice* out) {
+  if (!out) return fail(AN5D_E_INVALID, "null output");
+  AdjPlan ap;
+  int rc = plan_adjoint(p, cfg, ap);
+  if (rc) return rc;
+  AdjLaunch l{};
+  dim3 grid, block;
+  AdjFn fn = nullptr;
+  rc = adj_launch_plan(ap, ap.blocks[0], l, grid, block, fn);
+  if (rc) return rc;
+  const auto& vs = variants_of(p->stencil, p->dtype);
+  out->bt = ap.bt;
+  out->fwd_bt = ap.btf;
+  out->fwd_variant = 0;
+  while (out->fwd_variant < (int)vs.size() && vs[out->fwd_variant] != ap.fwd) out->fwd_variant++;
+  out->tile = -1;
+  for (int i = 0; i < kAdjTiles; i++)
+    if (ap.adj->tile[i].ck && ap.adj->tile[i].fn[ap.blocks[0]] == fn) out->tile = i;
+  out->columns = l.ntk;
+  out->segments = l.nseg;
   return AN5D_OK;
 }
 

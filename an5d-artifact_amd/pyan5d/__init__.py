@@ -390,6 +390,15 @@ def adjoint_host(name, u0, target, n, T, coefs=None, divisor=-1.0, bt=0, variant
     return loss.value, grad, gc, mf.value, mt.value
 
 
+def adjoint_resolve(name, n, T, dtype=np.float32, coefs=None, divisor=-1.0, bt=0, variant=-1, sl=0):
+    """The kernels an adjoint call runs (an5d_adjoint_resolve)."""
+    p, keep = make_problem(name, n, T, dtype, coefs, divisor)
+    cfg = make_config(bt, variant, sl)
+    out = (ctypes.c_int * 6)()
+    _check(lib().an5d_adjoint_resolve(ctypes.byref(p), ctypes.byref(cfg), out))
+    return dict(zip(("bt", "fwd_variant", "fwd_bt", "tile", "columns", "segments"), out))
+
+
 class AdjointWorkspace:
     """Device workspace for adjoint_device (checkpoints + two adjoint buffers)."""
 

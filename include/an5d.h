@@ -178,6 +178,14 @@ int an5d_init_grid(int dtype, void* A, long long cells, long long seed_base, int
  * bt=4 is about 75 GB); a size beyond the current device's memory is
  * rejected with AN5D_E_ALLOC and a message. */
 int an5d_adjoint_workspace(const an5d_problem* prob, const an5d_config* cfg, size_t* bytes);
+/* The kernels an adjoint call runs for `prob` and `cfg`: steps per block, the
+ * forward pass (variant, steps per launch), and the reverse block's first
+ * launch: register tile (an index, small grids first) or -1 for streams, and
+ * how many of them lie along dim 1 (columns) and dim 0 (segments). */
+typedef struct an5d_adjoint_choice {
+  int bt, fwd_variant, fwd_bt, tile, columns, segments;
+} an5d_adjoint_choice;
+int an5d_adjoint_resolve(const an5d_problem* prob, const an5d_config* cfg, an5d_adjoint_choice* out);
 /* Device form: enqueues on `stream`; *ms_fwd (optional) gets the time of the
  * checkpointed forward pass (synchronises on an event when non-NULL).
  * gcoef and loss are device doubles.  The workspace (size from

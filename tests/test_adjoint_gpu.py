@@ -248,5 +248,17 @@ def test_adjoint_block_deeper_than_the_tuned_forward_kernel(n):
             assert same_bits(gc, whole[2])
 
 
+@pytest.mark.parametrize("name,n,bt", [("star2d4r", [3700, 3900], 1), ("box2d3r", [2800, 2500], 1),
+                                       ("box2d4r", [4000, 1000], 1), ("star2d1r", [2000, 2000], 5)])
+def test_streams_that_hold_one_wave_fill_one_round(name, n, bt):
+    """FP64 reverse blocks whose kernel holds one wave a SIMD: as many segments as
+    one round of the chip's 1024 SIMDs takes, where they have 16 planes."""
+    c = pyan5d.adjoint_resolve(name, n, 24, np.float64)
+    print(f"case one round {name} {n} {c}", flush=True)
+    assert c["bt"] == bt and c["tile"] == -1
+    waves = c["columns"] * c["segments"]
+    assert 0.95 * 1024 < waves <= 1024
+
+
 def same_bits(a, b):
     return np.array_equal(a.view(np.uint64), b.view(np.uint64))
