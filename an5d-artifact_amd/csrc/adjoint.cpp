@@ -115,28 +115,33 @@ static int plan_adjoint(const an5d_problem* p, const an5d_config* cfg, AdjPlan& 
   if (!ap.adj) return fail(AN5D_E_UNSUPPORTED, "no adjoint kernels for this stencil/dtype");
   const auto& vs = variants_of(p->stencil, p->dtype);
   if (cfg && cfg->variant >= (int)vs.size()) return fail(AN5D_E_INVALID, "variant index out of range");
-  // forward kernel: the caller's variant, else the tuned/default forward choice
+  // forward kernel: the caller's variant, else the tuned/default forward choice.
+  // A register tile fitted to another size than its row's was chosen for the
+  // depth fitted with it, not for the block's few steps: past 48 MB the row's own
+  // shape (j2d5pt FP32 3700x3900, 24 steps: 868 -> 755 us; gradient2d 2800x2500
+  // 1047 -> 788; below, the fitted shape is up to 9 % the faster).
+  const bool own = !cfg || cfg->variant < 0;
+  const bool large = 2 * ap.g.area * (p->dtype == AN5D_FLOAT64 ? 8 : 4) > (48LL << 20);
   an5d_config fc{0, cfg ? cfg->variant : -1, 0, AN5D_EXACT};
   int bt_pref = 0, sl_pref = 0;
-  int rc = resolve(p, &fc, &ap.fwd, &bt_pref, &sl_pref);
+  int rc = resolve(p, &fc, &ap.fwd, &bt_pref, &sl_pref, large);
   if (rc) return rc;
   int bt = cfg && cfg->bt > 0 ? cfg->bt : ap.adj->btmax;
-  // a tuned choice that is shallower than the block (the one-step kernels) gives
-  // way to the stencil's sweep
-  if ((!cfg || cfg->variant < 0) && ap.fwd->btmax < bt && vs[0]->btmax >= bt) {
-    ap.fwd = vs[0];
-    bt_pref = bt;
-    sl_pref = 0;
-  }
-  // the block's few steps on a large FP32 grid are faster on the sweep than on a
-  // tile chosen for its depth (j2d9pt 3700x3900, 24 steps: 1145 -> 1001 us); not
-  // with a division (over 118, 4096^2, 64 steps: 3073 us on the tile, 3267)
-  const double divisor = p->divisor < 0 ? stencil_rt(p->stencil).divisor : p->divisor;
-  if (divisor == 0 && (!cfg || cfg->variant < 0) && ap.fwd->kind == kTile && p->dtype == AN5D_FLOAT32 &&
-      2 * ap.g.area * 4 > (48LL << 20) && vs[0]->kind == kSweep && vs[0]->btmax >= ap.adj->btmax && vs[0]->btmax >= bt) {
+  // blocks of one step on a large grid of radius 1: the sweep stores four
+  // intermediate states a launch, a tile one (star2d1r FP32 2800x2500, 24 steps:
+  // 894 us on the sweep, 1008 on the tile; at radius 2 they are equal)
+  if (own && large && ap.fwd->kind == kTile && bt < ap.adj->btmax && 4 * bt <= default_bt(stencil_rt(p->stencil), p->dtype) &&
+      vs[0]->kind == kSweep && vs[0]->btmax >= 4) {
     fc.variant = 0;
     rc = resolve(p, &fc, &ap.fwd, &bt_pref, &sl_pref);
     if (rc) return rc;
+  }
+  // a tuned choice that is shallower than the block (the one-step kernels) gives
+  // way to the stencil's sweep
+  if (own && ap.fwd->btmax < bt && vs[0]->btmax >= bt) {
+    ap.fwd = vs[0];
+    bt_pref = bt;
+    sl_pref = 0;
   }
   if (bt > ap.adj->btmax || bt > ap.fwd->btmax) {
     if (cfg && cfg->bt > 0) return fail(AN5D_E_UNSUPPORTED, "bt exceeds the adjoint or forward btmax");

@@ -591,7 +591,7 @@ static const Variant* deeper_variant(const an5d_problem* p, const std::vector<co
 }
 
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,
-            int* slout) {
+            int* slout, bool row_shape) {
   const auto& vs = variants_of(p->stencil, p->dtype);
   if (vs.empty()) return fail(AN5D_E_UNSUPPORTED, "no kernels compiled for this stencil/dtype");
   const StencilRT& s = stencil_rt(p->stencil);
@@ -611,7 +611,7 @@ int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout,
       v = vs[tc.variant];
       if (want_bt == 0) {
         want_bt = tc.bt;
-        if (!tc.same_size && v->kind == kTile) fit_tile(p, mode, vs, &v, &want_bt);
+        if (!tc.same_size && !row_shape && v->kind == kTile) fit_tile(p, mode, vs, &v, &want_bt);
       } else if (want_bt > tc.bt) {
         v = deeper_variant(p, vs, v, want_bt);
       }

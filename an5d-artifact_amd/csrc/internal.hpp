@@ -41,8 +41,10 @@ const StencilRT& stencil_rt(int id);
 const std::vector<const Variant*>& variants_of(int stencil, int dtype);
 bool make_geom(const an5d_problem* p, Geom& g, std::string& err);
 an5d_layout reference_layout(const Geom& g);
+// row_shape: a register tile that a table row of another size names stays as it is
 int resolve(const an5d_problem* p, const an5d_config* cfg, const Variant** vout, int* btout,
-            int* slout);
+            int* slout, bool row_shape = false);
+int default_bt(const StencilRT& s, int dtype);
 // plan_launch's mode: AN5D_EXACT, AN5D_FAST, or kLaunchShare (exact, the
 // shared-product kernels)
 constexpr int kLaunchShare = 2;

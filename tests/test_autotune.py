@@ -91,6 +91,29 @@ def test_callers_depth_beyond_the_rows(tmp_path):
     pyan5d.tune_clear()
 
 
+def test_adjoint_forward_pass_on_a_rows_tile(tmp_path):
+    """A row that names a register tile: the adjoint's forward pass takes its
+    shape on large grids, with and without a division; single steps of radius 1
+    take the sweep, which stores four states a launch."""
+    path = tmp_path / "t.tsv"
+    for name, bt in (("gradient2d", 2), ("j2d5pt", 5), ("j2d9pt", 3)):
+        vs = pyan5d.variants(name, 0)
+        row = [v for v in vs if v["kind"] == 5][-1]
+        path.write_text(f"{name} 0 0 4096 4096 0 {row['index']} 5 0 1.0\n")
+        pyan5d.tune_clear()
+        pyan5d.tune_load(str(path))
+        for n in ([4096, 4096], [3700, 3900], [2800, 2500], [6000, 9000]):
+            for div in (-1.0,) if name == "gradient2d" else (-1.0, 0.0, 7.0):
+                c = pyan5d.adjoint_resolve(name, n, 24, np.float32, divisor=div)
+                assert (c["bt"], c["fwd_variant"], c["fwd_bt"]) == (bt, row["index"], bt), (name, n, div, c)
+            c = pyan5d.adjoint_resolve(name, n, 24, np.float32, bt=1)
+            if name == "j2d9pt":
+                assert (c["bt"], c["fwd_variant"], c["fwd_bt"]) == (1, row["index"], 1)
+            else:
+                assert (c["bt"], c["fwd_variant"], c["fwd_bt"]) == (1, 0, 4)
+    pyan5d.tune_clear()
+
+
 def test_tune_table_records_register_cap(tmp_path):
     """The cap column: a capped twin's deep block reports its cap, its
     shallow blocks (which share the uncapped kernels) report none."""
