@@ -131,6 +131,7 @@ using namespace an5d;
 
 struct an5d_batch {
   bool adjoint = false;
+  bool streams = false;  // forward batch: wave tiles from a counter, else a workgroup per register tile
   int n = 0;
   int levels = 0;
   int sl = kDefaultSl;
@@ -143,7 +144,8 @@ struct an5d_batch {
   BatchUnit* d_units = nullptr;
   std::vector<long long> rec_off, unit_off;
   std::vector<int> nfwd, nadj;
-  int* d_counters = nullptr;  // adjoint batch: two per level
+  int* d_counters = nullptr;  // streams and the adjoint batch: two per level
+  int counters_cap = 0;       // levels the counter array holds
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipStream_t cap = nullptr;
@@ -248,7 +250,8 @@ bool level_recs(const an5d_batch* b, const Inst& I, int m, std::vector<BatchRec>
     r.dst = static_cast<char*>(I.dA) + (size_t)((m + 1) % 2) * gbytes;
     r.s0 = I.g.D2;
     r.bt = k;
-    tile_tiling(I, k, r);
+    if (b->streams) fwd_tiling(I, k, sl, r);
+    else tile_tiling(I, k, r);
     recs.push_back(r);
     return true;
   }
@@ -355,7 +358,7 @@ void place_chains(an5d_batch* b) {
 }
 
 double rec_cost(const an5d_batch* b, const BatchRec& r) {
-  if (!b->adjoint) return r.bt;  // tiles of one size
+  if (!b->adjoint && !b->streams) return r.bt;  // tiles of one size
   const double cells = (double)r.sl * 64.0 * batch_ck();
   if (r.type == kUnitAdj) return 2.0 * cells * r.bt;
   if (r.type == kUnitFwd) return cells * r.bt;
@@ -400,7 +403,7 @@ int build_levels(an5d_batch* b) {
         const long long nt = (long long)r.ntk * r.nseg;
         // tiles by the XCD that runs them (workgroups go round-robin over 8):
         // neighbours, which read each other's halo, share its L2
-        const long long q = b->adjoint ? 0 : nt / 8;
+        const long long q = b->adjoint || b->streams ? 0 : nt / 8;
         for (long long t = 0; t < nt; t++) units.push_back(BatchUnit{rid, (int)(t < 8 * q ? t % 8 * q + t / 8 : t)});
         nu += nt;
       }
@@ -474,17 +477,60 @@ int prior_bt(const Inst& I) {
   return best;
 }
 
+// Streams for a forward batch whose levels fill the chip with them, where they do
+// less work per cell than register tiles.  ns per 1000 cell-steps, streams at five
+// steps a launch / tiles at their own depth, 400 M and 138 M cells in a level:
+//   j2d5pt over 118 0.54/0.72, 0.66/0.73; over 7 0.74/0.95; undivided 0.74/0.59
+//   j2d9pt over 118 0.87/1.21, 0.92/1.22; over 7 1.17/1.45; undivided 1.17/1.08
+//   j2d9pt-gol over 118 0.77/0.99, 0.83/1.00; undivided 1.02/0.83
+//   star2d2r 0.64/1.06, 0.69/1.07; over 7 1.03/1.34
+// with fewer cells the streams take about 16 / (M cells) more (64 M: 0.80/0.75,
+// 1.15/1.28, 1.09/1.02 and 0.90/1.07 in the same order), so the line lies at
+// 100 M, for the two stencils of nine points and a divisor at 200 M (at three steps,
+// 138 M: 1.24/1.22 and 1.13/1.10).  At a caller's three steps streams are also
+// ahead undivided (0.79/0.95, 1.10/1.21, 0.97/1.08), at one and two the tiles are
+// (2.4/3.2, 1.4/1.7).
+bool prefer_streams(const an5d_batch* b) {
+  auto work = [](const Inst& I) { return (double)(I.g.D0 - 2 * I.g.r) * (I.g.D2 - 2 * I.g.r) * I.T; };
+  double total = 0, favoured = 0;
+  int longest = 0;
+  for (const Inst& I : b->inst) {
+    total += work(I);
+    if (I.T > longest) longest = I.T;
+  }
+  if (longest == 0) return false;
+  const double cells = total / longest;  // of a level, on average
+  for (const Inst& I : b->inst) {
+    const StencilRT& s = stencil_rt(I.stencil);
+    const bool star2 = s.rad == 2 && s.divisor == 0;
+    if (I.bt_fixed != 0 && I.bt_fixed < 3) continue;
+    if (!I.has_div && !star2 && I.bt_fixed != 3) continue;
+    if (cells >= (star2 || s.ntaps <= 5 ? 100e6 : 200e6)) favoured += work(I);
+  }
+  return 2 * favoured > total;
+}
+
 // Forward batch: every instance's launch schedule under the batch's bt
-// policy, the chains placed.
-void plan_forward(an5d_batch* b) {
+// policy, the chains placed, the counters sized.
+int plan_forward(an5d_batch* b) {
   for (Inst& I : b->inst) {
     int bt = I.bt_fixed > 0 ? I.bt_fixed : (b->bt_policy > 0 ? b->bt_policy : I.bt_prior);
-    if (bt > tile_max_bt(I.g.r)) bt = tile_max_bt(I.g.r);
+    const int most = b->streams ? batch_max_bt() : tile_max_bt(I.g.r);
+    if (bt > most) bt = most;
     const int nl = an5d_schedule(I.T, bt, nullptr, 0);
     I.steps.resize(nl);
     an5d_schedule(I.T, bt, I.steps.data(), nl);
   }
   place_chains(b);
+  if (b->streams && b->levels > b->counters_cap) {
+    (void)hipFree(b->d_counters);
+    b->d_counters = nullptr;
+    b->counters_cap = 0;
+    const hipError_t e = hipMalloc(&b->d_counters, sizeof(int) * 2 * b->levels);
+    if (e != hipSuccess) return fail(AN5D_E_ALLOC, "hipMalloc(batch counters)");
+    b->counters_cap = b->levels;
+  }
+  return AN5D_OK;
 }
 
 }  // namespace
@@ -510,11 +556,12 @@ extern "C" int an5d_batch_create(an5d_batch** out, int n, const an5d_problem* pr
       return fail(AN5D_E_UNSUPPORTED, "batched bt is at most " + std::to_string(batch_max_bt()));
     }
     I.bt_fixed = bt;
-    I.bt_prior = bt > 0 ? bt : prior_bt(I);
     I.sl_fixed = (cfgs && cfgs[i].sl > 0) ? cfgs[i].sl : 0;
   }
-  plan_forward(b);
-  int rc = build_levels(b);
+  b->streams = prefer_streams(b);
+  for (Inst& I : b->inst) I.bt_prior = I.bt_fixed > 0 ? I.bt_fixed : (b->streams ? batch_max_bt() : prior_bt(I));
+  int rc = plan_forward(b);
+  if (rc == AN5D_OK) rc = build_levels(b);
   if (rc) { batch_free(b); return rc; }
   *out = b;
   return AN5D_OK;
@@ -635,6 +682,7 @@ extern "C" int an5d_batch_adjoint_create(an5d_batch** out, int n, const an5d_pro
   place_chains(b);
   hipError_t e = hipMalloc(&b->d_counters, sizeof(int) * 2 * (b->levels > 0 ? b->levels : 1));
   if (e != hipSuccess) { batch_free(b); return fail(AN5D_E_ALLOC, "hipMalloc(batch counters)"); }
+  b->counters_cap = b->levels;
   e = hipDeviceSynchronize();
   if (e != hipSuccess) { batch_free(b); return hip_fail(e, "batch workspace clear"); }
   int rc = build_levels(b);
@@ -665,7 +713,9 @@ extern "C" int an5d_batch_run(an5d_batch* b, void* stream) {
       const int occ = batch_occupancy(kind);
       return occ > 0 && cus > 0 ? (long long)occ * cus : 2048LL;
     };
-    const long long res_f = b->adjoint ? resident(kLevelFwdMisc) : 0, res_a = b->adjoint ? resident(kLevelAdj) : 0;
+    const bool counted = b->adjoint || b->streams;
+    const int kf = b->adjoint ? kLevelFwdMisc : kLevelFwd;
+    const long long res_f = counted ? resident(kf) : 0, res_a = b->adjoint ? resident(kLevelAdj) : 0;
     auto grid_of = [](long long units, long long res) {
       long long g = cdiv(units, 4);  // four waves per workgroup, one unit each at first
       if (g > res) g = res;
@@ -673,17 +723,17 @@ extern "C" int an5d_batch_run(an5d_batch* b, void* stream) {
     };
     e = hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
-    hipError_t le = b->adjoint ? batch_launch_reset(b->d_counters, 2 * b->levels, b->cap) : hipSuccess;
+    hipError_t le = counted ? batch_launch_reset(b->d_counters, 2 * b->levels, b->cap) : hipSuccess;
     for (int l = 0; l < b->levels && le == hipSuccess; l++) {
       const BatchRec* recs = b->d_recs + b->rec_off[l];
       const BatchUnit* uf = b->d_units + b->unit_off[l];
       const BatchUnit* ua = uf + b->nfwd[l];
-      if (!b->adjoint) {
+      if (!counted) {
         if (b->nfwd[l] > 0) le = batch_launch_tiles(recs, uf, b->nfwd[l], b->cap);
         continue;
       }
       if (b->nfwd[l] > 0)
-        le = batch_launch_level(kLevelFwdMisc, recs, uf, b->nfwd[l], b->d_counters + 2 * l, grid_of(b->nfwd[l], res_f),
+        le = batch_launch_level(kf, recs, uf, b->nfwd[l], b->d_counters + 2 * l, grid_of(b->nfwd[l], res_f),
                                 b->cap);
       if (le == hipSuccess && b->nadj[l] > 0)
         le = batch_launch_level(kLevelAdj, recs, ua, b->nadj[l], b->d_counters + 2 * l + 1,
@@ -736,11 +786,14 @@ extern "C" int an5d_batch_tune(an5d_batch* b, int reps, int* best_sl, double* be
   int best = b->sl, best_pol = b->bt_policy;
   double best_t = -1.0;
   int rc = AN5D_OK;
-  // forward batch: bt policy (each instance's own, or one bt for all); the
-  // forward + adjoint batch keeps its blocks and tries segment lengths
+  // forward batch: bt policy (each instance's own, or one bt for all), on streams
+  // with segment lengths; the forward + adjoint batch keeps its blocks and tries
+  // segment lengths
   std::vector<int> policies = {b->bt_policy};
   std::vector<int> sls(kSlCandidates, kSlCandidates + sizeof(kSlCandidates) / sizeof(int));
-  if (!b->adjoint) {
+  if (b->streams) {
+    policies = {0, 3, 4};
+  } else if (!b->adjoint) {
     policies = {0, 4, 6, 8};
     sls = {b->sl};
   }
@@ -749,7 +802,8 @@ extern "C" int an5d_batch_tune(an5d_batch* b, int reps, int* best_sl, double* be
     b->sl = sl;
     if (!b->adjoint && pol != b->bt_policy) {
       b->bt_policy = pol;
-      plan_forward(b);
+      rc = plan_forward(b);
+      if (rc) break;
     }
     rc = build_levels(b);
     if (rc) break;
@@ -784,7 +838,8 @@ extern "C" int an5d_batch_tune(an5d_batch* b, int reps, int* best_sl, double* be
   b->sl = best;
   if (!b->adjoint && best_pol != b->bt_policy) {
     b->bt_policy = best_pol;
-    plan_forward(b);
+    rc = plan_forward(b);
+    if (rc) return rc;
   }
   rc = build_levels(b);
   if (rc) return rc;

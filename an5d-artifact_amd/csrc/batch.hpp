@@ -11,8 +11,9 @@
 // a HIP graph.
 //
 // Unit types:
-//   FWD    one wave tile of a forward launch (the sweep of sweep.hpp); in the
-//          forward batch one workgroup tile (tile2.hpp), no counter
+//   FWD    one wave tile of a forward launch (the sweep of sweep.hpp); in a
+//          forward batch that does not fill the chip with those one workgroup
+//          tile (tile2.hpp), no counter
 //   ADJ    one wave tile of a reverse block (the adjoint of adjoint.hpp)
 //   PREP   rows of the initial state copied into checkpoint slot 0, with the
 //          halo cells of those rows copied into every other slot (the sweeps
@@ -59,7 +60,7 @@ struct BatchUnit {
 };
 
 // level kernel kinds (see batch_level_kernel)
-constexpr int kLevelFwdMisc = 0, kLevelAdj = 1;
+constexpr int kLevelFwd = 0, kLevelFwdMisc = 1, kLevelAdj = 2;
 
 // Stencils the batched kernels are built for (2D, FP32): forward CK = 4, the
 // adjoint at its own FP32 shape (CK = 4 for radius <= 2).
@@ -270,10 +271,11 @@ __device__ __forceinline__ void batch_tile_dispatch(float (&u)[kTileCJ][kTileCK]
   batch_tile_steps<K, -1>(u, lds, p, r, lane, w);
 }
 
-// A level of the forward batch: one workgroup per register tile (tile2.hpp) of
-// every instance.  Bound by vector issue, as a launch of one large grid is.  On
-// the streamed sweep's wave tiles a level of 24 instances had one or two waves a
-// SIMD and stopped at five steps.
+// A level of the forward batch on register tiles: one workgroup per tile
+// (tile2.hpp) of every instance.  On the streamed sweep's wave tiles a level of 24
+// instances had one or two waves a SIMD and stopped at five steps; levels that
+// fill the chip with streams take those where they do less work per cell
+// (batch.cpp: prefer_streams).
 __global__ __launch_bounds__(64 * kTileNW, 5) void batch_tile_kernel(const BatchRec* __restrict__ recs,
                                                                   const BatchUnit* __restrict__ units) {
   extern __shared__ __align__(16) unsigned char an5d_lds[];
@@ -295,9 +297,10 @@ __global__ __launch_bounds__(64 * kTileNW, 5) void batch_tile_kernel(const Batch
   tile2_store<float, kTileCK, kTileCJ>(u, p, static_cast<float*>(r.dst), r.s0);
 }
 
-// Level kernels of the forward + adjoint batch, each with its own register
-// budget: one runs its FWD, PREP, SEED, GRAD and FINISH units, the other its ADJ
-// units.  Every wave leaves the loop once the counter passes nunits.
+// Level kernels, each with its own register budget: KIND 0 runs FWD units (the
+// streams of a forward batch), KIND 1 the FWD, PREP, SEED, GRAD and FINISH units
+// of the forward + adjoint batch, KIND 2 its ADJ units.  Every wave leaves the
+// loop once the counter passes nunits.
 template <int KIND>
 __global__ __launch_bounds__(64 * kBatchNW) void batch_level_kernel(const BatchRec* __restrict__ recs,
                                                                     const BatchUnit* __restrict__ units,
@@ -325,7 +328,7 @@ __global__ __launch_bounds__(64 * kBatchNW) void batch_level_kernel(const BatchR
           case 2: batch_fwd_dispatch<2>(r, wu.tile); break;
           default: batch_fwd_dispatch<3>(r, wu.tile); break;
         }
-      } else {
+      } else if constexpr (KIND == kLevelFwdMisc) {
         if (r.type == kUnitPrep) batch_prep(r, wu.tile);
         else if (r.type == kUnitSeed) batch_seed(r, wu.tile);
         else if (r.type == kUnitGrad) batch_grad(r, wu.tile);

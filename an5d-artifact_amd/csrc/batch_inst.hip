@@ -8,7 +8,8 @@ namespace an5d {
 
 static const void* level_kernel(int kind) {
   if (kind == kLevelAdj) return reinterpret_cast<const void*>(&batch_level_kernel<kLevelAdj>);
-  return reinterpret_cast<const void*>(&batch_level_kernel<kLevelFwdMisc>);
+  if (kind == kLevelFwdMisc) return reinterpret_cast<const void*>(&batch_level_kernel<kLevelFwdMisc>);
+  return reinterpret_cast<const void*>(&batch_level_kernel<kLevelFwd>);
 }
 
 hipError_t batch_launch_level(int kind, const BatchRec* recs, const BatchUnit* units, int nunits,
@@ -16,9 +17,12 @@ hipError_t batch_launch_level(int kind, const BatchRec* recs, const BatchUnit* u
   if (kind == kLevelAdj)
     hipLaunchKernelGGL(batch_level_kernel<kLevelAdj>, dim3(grid), dim3(64 * kBatchNW), 0, st, recs, units,
                        nunits, counter);
-  else
+  else if (kind == kLevelFwdMisc)
     hipLaunchKernelGGL(batch_level_kernel<kLevelFwdMisc>, dim3(grid), dim3(64 * kBatchNW), 0, st, recs,
                        units, nunits, counter);
+  else
+    hipLaunchKernelGGL(batch_level_kernel<kLevelFwd>, dim3(grid), dim3(64 * kBatchNW), 0, st, recs, units,
+                       nunits, counter);
   return hipGetLastError();
 }
 

@@ -464,7 +464,8 @@ def adjoint_device_noalloc(name, u0, target, grad, gcoef, loss, n, T, coefs=None
 class Batch:
     """Batched forward over many device grids (an5d_batch_create).  `items` is
     a list of (name, n, T, tensor[2, ...], coefs, divisor); bt / sl apply to
-    every item (0: the depth of least cost; the forward batch has no segments)."""
+    every item (0: the depth of least cost / the batch-wide segment length;
+    register tiles have no segments)."""
 
     def __init__(self, items, bt=0, sl=0):
         n = len(items)
@@ -494,8 +495,8 @@ class Batch:
         _check(lib().an5d_batch_run(self.handle, _stream_ptr(stream)))
 
     def tune(self, reps=2):
-        """Measured choice of the depth (forward) or the batch-wide segment
-        length (forward + adjoint); returns (sl, ms)."""
+        """Measured choice of the depth (forward) and the batch-wide segment
+        length (streams, forward + adjoint); returns (sl, ms)."""
         sl, ms = ctypes.c_int(), ctypes.c_double()
         _check(lib().an5d_batch_tune(self.handle, int(reps), ctypes.byref(sl), ctypes.byref(ms)))
         self._info()

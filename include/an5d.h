@@ -222,8 +222,9 @@ int an5d_adjoint_host(const an5d_problem* prob, const void* u0, const void* targ
  * star2d2r and j2d9pt-gol; any sizes and timesteps.
  *
  * Each instance's work is a chain of levels; one kernel launch covers one
- * level of every instance: a workgroup per tile in the forward batch, waves
- * pulling (instance, tile) work units from a device counter in the forward +
+ * level of every instance: a workgroup per register tile in a forward batch,
+ * waves pulling (instance, tile) work units from a device counter where its
+ * levels are large enough to fill the chip with streams, and in the forward +
  * adjoint batch.  The whole level sequence is captured into one HIP graph on
  * the first run (replayed afterwards).  Chains are placed on the level axis so
  * that the estimated work per level is even.
@@ -231,8 +232,8 @@ int an5d_adjoint_host(const an5d_problem* prob, const void* u0, const void* targ
  * an5d_batch_create: forward only.  dA[i] holds both buffers of instance i
  * (reference layout); after a run buffer T_i%2 holds u_T, bit for bit the
  * single-grid result.  cfgs (optional): per-instance bt (<= 5; 0: the
- * depth of least cost for the instance's tiles) and sl (accepted; the forward
- * batch has no segments).
+ * depth of least cost for the instance's tiles, 5 on streams) and sl (the
+ * streams' segment length, 0: batch-wide; tiles have no segments).
  *
  * an5d_batch_adjoint_create: forward + adjoint.  Currently switched off: it
  * returns AN5D_E_UNSUPPORTED (its first GPU run stalled; cause not found).
@@ -251,8 +252,9 @@ int an5d_adjoint_host(const an5d_problem* prob, const void* u0, const void* targ
  *
  * an5d_batch_tune: times the level sequence (`reps` replays each) and keeps the
  * fastest: for a forward batch over bt policies (each instance's own bt, or
- * bt = 4, 6, 8 for all instances without a caller bt), for a forward + adjoint
- * batch over batch-wide segment lengths (32-256); a forward batch's grids are
+ * bt = 4, 6, 8, on streams 3, 4, for all instances without a caller bt), on
+ * streams and in a forward + adjoint batch over batch-wide segment lengths
+ * (32-256); a forward batch's grids are
  * restored afterwards.  an5d_batch_run: enqueue one run on
  * `stream` (a hipStream_t); runs that overlap on one batch race. */
 typedef struct an5d_batch an5d_batch;

@@ -286,3 +286,50 @@ def test_batch_tiles_at_their_edges(torch_cuda, bt):
         O.run(name, ref, n, T, divisor=div)
         assert _same_bits(it[3][T % 2].cpu().numpy(), ref[T % 2]), (name, n, T, div)
     b.close()
+
+
+def test_large_batch_on_streams(torch_cuda):
+    """A batch whose levels fill the chip takes streams (by its count of work
+    units): every division form, a grid of few cells, one without steps, odd step
+    counts; each instance bit for bit the single grid's one-step launches, the
+    small one the oracle's; twice, and once more after the tuner."""
+    torch = torch_cuda
+    specs = [("star2d2r", [8400, 6144], 9, -1.0), ("j2d5pt", [6144, 6001], 6, 118.0), ("star2d2r", [4000, 4096], 7, 3.0),
+             ("j2d9pt", [3000, 4096], 9, 118.0), ("j2d9pt-gol", [2000, 3000], 5, 7.0), ("j2d5pt", [5, 7], 9, 0.0),
+             ("j2d9pt", [40, 60], 0, -1.0)]
+    items, refs = [], []
+    for i, (name, n, T, div) in enumerate(specs):
+        r = O.info(name)["rad"]
+        g = torch.Generator(device="cuda").manual_seed(i)
+        u = torch.rand([x + 2 * r for x in n], device="cuda", generator=g)
+        t = torch.stack([u, u])
+        ref = t.clone()
+        pyan5d.forward_device(name, ref, n, T, divisor=div, bt=1)
+        items.append((name, n, T, t, None, div))
+        refs.append(ref[T % 2])
+    inputs = [it[3].clone() for it in items]
+    b = pyan5d.Batch(items)
+    units = 0
+    for (name, n, T, _) in specs:
+        r = O.info(name)["rad"]
+        for k in pyan5d.schedule(T, 5):
+            units += -(-n[1] // (256 - 2 * k * r)) * -(-n[0] // min(64, n[0]))
+    assert b.units == units
+    for rep in range(3):
+        for it, a in zip(items, inputs):
+            it[3].copy_(a)
+        torch.cuda.synchronize()
+        print(f"case batch on streams, run {rep}", flush=True)
+        if rep == 2:
+            b.tune(reps=1)
+        b.run()
+        torch.cuda.synchronize()
+        for it, ref in zip(items, refs):
+            assert torch.equal(it[3][it[2] % 2].view(torch.int32), ref.view(torch.int32)), (it[0], it[1], rep)
+    small = inputs[5].cpu().numpy()
+    O.run("j2d5pt", small, [5, 7], 9, divisor=0.0)
+    assert _same_bits(refs[5].cpu().numpy(), small[1])
+    b.close()
+    few = pyan5d.Batch(items[4:])  # a few cells: register tiles
+    assert few.units < units // 8
+    few.close()
