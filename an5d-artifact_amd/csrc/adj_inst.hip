@@ -64,14 +64,15 @@ int occupancy(int bt) {
 }
 
 // Register-tile shapes (adj_tile.hpp), FP64 stencils of up to 25 taps: 16 waves
-// of few cells for the smallest grids, 8 waves (whose 256 registers hold the
-// block's states, and less halo) above.  Left out: 16 waves for the box of
-// radius 2 (spills: 3199 us against 769 on 8 waves for 60 steps of 256^2); at
-// radius 3-4 the edge rows of a larger tile exceed LDS.
+// of few cells for the smallest grids of radius 1, 8 waves (whose 256 registers
+// hold the block's states, and less halo) above.  At radius 2 the 8 waves alone: 16
+// of half their cells cover the same tile and are slower (60 steps of 256^2: j2d9pt
+// 546 us against 465; the box spills, 3199 against 769); at radius 3-4 the edge
+// rows of a larger tile than the first exceed LDS.
 template <int I>
 constexpr bool adj_tiled() {
   if (!AN5D_F64 || !D::linear || D::ntaps > 25) return false;
-  return I == 0 ? D::ntaps <= 9 || D::rad >= 3 : D::rad <= 2;
+  return I == 0 ? D::rad != 2 : D::rad <= 2;
 }
 template <int I> constexpr int tile_ck() { return D::rad >= 3 ? 4 : (I == 0 && D::rad == 1 ? 1 : 2); }
 template <int I> constexpr int tile_cj() { return I == 0 ? 2 : 4; }

@@ -311,6 +311,8 @@ static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, d
         if (share_of(nseg) > 12) break;
       }
     }
+    // against the tiles a lone wave, whose latency nothing covers, counts as two
+    if (held == 1) t_best *= 2;
   }
   l.D0 = (int)ap.g.D0;
   l.D2 = (int)ap.g.D2;

@@ -260,5 +260,27 @@ def test_streams_that_hold_one_wave_fill_one_round(name, n, bt):
     assert 0.95 * 1024 < waves <= 1024
 
 
+@pytest.mark.parametrize("name,n,tile", [
+    ("star2d1r", [150, 310], 0), ("j2d9pt-gol", [150, 310], 0), ("star2d2r", [150, 310], 1), ("j2d9pt", [150, 310], 1),
+    ("box2d2r", [150, 310], 1), ("star2d3r", [150, 310], 0), ("star2d4r", [150, 310], 0), ("star2d1r", [600, 620], 1),
+    ("box2d1r", [600, 620], 1), ("j2d5pt", [600, 620], 1), ("j2d9pt-gol", [600, 620], 1), ("star2d2r", [600, 620], 1)])
+def test_reverse_tile_of_the_plan(name, n, tile):
+    """Each register tile of the FP64 reverse block, by the plan's choice: 16 waves
+    for small grids of radius 1 and at radius 3-4, 8 waves at radius 2 and from
+    about 550^2 on; several tiles with remainders in both directions and a short
+    last block, against the FP64 oracle."""
+    bt = adj_btmax(name, np.float64)
+    T = 2 * bt + 1
+    c = pyan5d.adjoint_resolve(name, n, T, np.float64)
+    print(f"case reverse tile {name} {n} {c}", flush=True)
+    assert c["tile"] == tile and c["columns"] > 1 and c["segments"] > 1
+    u0, target, co, div = problem(name, n, np.float64, seed=sum(n))
+    loss, g, gc, _, _ = pyan5d.adjoint_host(name, u0, target, n, T, coefs=co, divisor=div)
+    oloss, og, ogc = O.adjoint(name, u0, target, n, T, coefs=co, divisor=div)
+    assert abs(loss - oloss) <= 1e-10 * oloss
+    for a, o in ((g, og), (gc, ogc)):
+        assert np.max(np.abs(a - o)) <= 1e-10 * np.max(np.abs(o))
+
+
 def same_bits(a, b):
     return np.array_equal(a.view(np.uint64), b.view(np.uint64))
