@@ -333,3 +333,34 @@ def test_large_batch_on_streams(torch_cuda):
     few = pyan5d.Batch(items[4:])  # a few cells: register tiles
     assert few.units < units // 8
     few.close()
+
+
+def test_batch_tiles_at_their_own_depth(torch_cuda):
+    """Register tiles of a batch at the depth of least cost (six steps and more)
+    and at the tuner's: several tiles with remainders, every stencil and division
+    form; each instance bit for bit the oracle."""
+    torch = torch_cuda
+    rng = np.random.default_rng(23)
+    items, hosts = [], []
+    for name, div in [("j2d5pt", 118.0), ("j2d5pt", 0.0), ("j2d9pt", 118.0), ("j2d9pt", 3.0), ("star2d2r", -1.0),
+                      ("j2d9pt-gol", 7.0), ("j2d9pt-gol", 118.0)]:
+        r = O.info(name)["rad"]
+        n = [201, 287]
+        u = rng.random([x + 2 * r for x in n]).astype(np.float32)
+        hosts.append((name, n, 33, div, np.stack([u, u])))
+        items.append((name, n, 33, torch.from_numpy(hosts[-1][4].copy()).cuda(), None, div))
+    b = pyan5d.Batch(items)
+    assert b.levels <= 33 // 5
+    for tuned in (False, True):
+        print(f"case batch tiles at their own depth, tuned {tuned}, levels {b.levels}", flush=True)
+        if tuned:
+            for (_, _, _, _, A), it in zip(hosts, items):
+                it[3].copy_(torch.from_numpy(A))
+            b.tune(reps=1)
+        b.run()
+        torch.cuda.synchronize()
+        for (name, n, T, div, A), it in zip(hosts, items):
+            ref = A.copy()
+            O.run(name, ref, n, T, divisor=div)
+            assert _same_bits(it[3][T % 2].cpu().numpy(), ref[T % 2]), (name, div)
+    b.close()

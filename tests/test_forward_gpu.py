@@ -617,3 +617,64 @@ def test_segments_of_large_grids_fill_one_round(name, dt, mode, bt, n, ck, waves
     sl = pyan5d.resolve_config(name, n, dt, mode=mode, bt=bt, variant=0)["sl"]
     runs = -(-n[0] // sl) * -(-n[1] // (64 * ck - 2 * bt * r))
     assert 0.9 * waves * 1024 <= runs <= waves * 1024
+
+
+def fma_bound(name, dt, A, n, T, div):
+    """How far FMA mode may lie from the C loop after T steps (linear stencils),
+    from the unit roundoff u: a step's products, sums and division round ntaps + 1
+    times, and so do the folded coefficients and the chained FMAs, each time by u
+    times sum |c v| at most, and a step passes on the difference that it finds
+    times sum |c| / divisor.  The field's bound is the oracle's largest value."""
+    taps, c = O.taps(name)
+    d = O.info(name)["divisor"] if div < 0 else div
+    S = float(np.sum(np.abs(np.asarray(c, dtype=np.float64)))) / (d or 1.0)
+    u = 2.0 ** -24 if dt == np.float32 else 2.0 ** -53
+    err, M = 0.0, float(np.max(np.abs(A)))
+    for _ in range(T):
+        err = S * err + 1.01 * 2 * (len(taps) + 1) * u * S * (M + err)
+        M *= max(1.0, S)
+    return err
+
+
+@pytest.mark.parametrize("name", TILE_NAMES + ["star3d1r", "box3d1r", "j3d27pt"])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_register_tiles_in_fma_mode(name, dt):
+    """Every register-tile kernel (kind 5) in FMA mode: several tiles with
+    remainders, a shallow and the deepest block, the source's divisor and another;
+    within the rounding bound of the C loop, gradient2d (which has no FMA form) bit
+    for bit."""
+    r = O.info(name)["rad"]
+    dim = O.info(name)["dim"]
+    for v in pyan5d.variants(name, 0 if dt == np.float32 else 1):
+        if v["kind"] != 5:
+            continue
+        th, tw = v["nw"] * v["cj"] - 2 * r, 64 * v["ck"] - 2 * r
+        for bt in sorted({min(2, v["btmax"]), v["btmax"]}):
+            for div in (-1.0, 7.0) if name != "gradient2d" else (-1.0,):
+                n = [2 * th + 5, tw + 70] if dim == 2 else [19, 2 * th + 1, 130]
+                T = bt + 2
+                print(f"case tiles FMA {name} {np.dtype(dt).name} variant {v['index']} bt={bt} n={n} divisor={div}",
+                      flush=True)
+                A = rand_grid(name, n, dt, seed=sum(n) + bt)
+                B = A.copy()
+                pyan5d.forward_host(name, A, n, T, variant=v["index"], bt=bt, divisor=div, mode=pyan5d.FAST)
+                tol = 0.0 if name == "gradient2d" else fma_bound(name, dt, B, n, T, div)
+                O.run(name, B, n, T, divisor=div)
+                got, ref = A[T % 2].astype(np.float64), B[T % 2].astype(np.float64)
+                assert np.max(np.abs(got - ref)) <= tol
+
+
+def test_box3d_rows_shorter_than_a_run_beside_a_row_of_columns():
+    """A grid whose nearest table row names the column kernel, but whose rows are
+    shorter than a lane's run: the default path takes the direct kernel, one cell
+    more the columns."""
+    name, T = "box3d2r", 2
+    for n, kind in (([500, 600, 3], 1), ([500, 600, 4], 4)):
+        c = pyan5d.resolve_config(name, n, np.float64)
+        print("case columns beside a row", name, n, c, flush=True)
+        assert pyan5d.variants(name, 1)[c["variant"]]["kind"] == kind
+        A = rand_grid(name, n, np.float64, seed=5)
+        B = A.copy()
+        pyan5d.forward_host(name, A, n, T)
+        O.run(name, B, n, T)
+        assert same(A[T % 2], B[T % 2])
