@@ -477,6 +477,27 @@ int prior_bt(const Inst& I) {
   return best;
 }
 
+// The same on streams: a launch's cost by its steps, ns per 1000 cells (j2d5pt over
+// 118; star2d2r's are in proportion).  One of one or two steps, which the end of a
+// schedule may have, takes longer than one of five: 64 steps take 16 launches of
+// four or 12 of five and two of two, 38.6 and 41.8.
+int stream_bt(const Inst& I) {
+  constexpr double kCost[kBatchMaxBT + 1] = {0, 3.2, 3.3, 2.3, 2.4, 2.9};
+  int best = kBatchMaxBT;
+  double best_c = 1e300;
+  for (int bt = kBatchMaxBT; bt >= 3; bt--) {
+    std::vector<int> steps(an5d_schedule(I.T, bt, nullptr, 0));
+    an5d_schedule(I.T, bt, steps.data(), (int)steps.size());
+    double c = 0;
+    for (int k : steps) c += kCost[k];
+    if (c < best_c) {
+      best_c = c;
+      best = bt;
+    }
+  }
+  return best;
+}
+
 // Streams for a forward batch whose levels fill the chip with them, where they do
 // less work per cell than register tiles.  ns per 1000 cell-steps, streams at five
 // steps a launch / tiles at their own depth, 400 M and 138 M cells in a level:
@@ -559,7 +580,7 @@ extern "C" int an5d_batch_create(an5d_batch** out, int n, const an5d_problem* pr
     I.sl_fixed = (cfgs && cfgs[i].sl > 0) ? cfgs[i].sl : 0;
   }
   b->streams = prefer_streams(b);
-  for (Inst& I : b->inst) I.bt_prior = I.bt_fixed > 0 ? I.bt_fixed : (b->streams ? batch_max_bt() : prior_bt(I));
+  for (Inst& I : b->inst) I.bt_prior = I.bt_fixed > 0 ? I.bt_fixed : (b->streams ? stream_bt(I) : prior_bt(I));
   int rc = plan_forward(b);
   if (rc == AN5D_OK) rc = build_levels(b);
   if (rc) { batch_free(b); return rc; }

@@ -232,7 +232,7 @@ int an5d_adjoint_host(const an5d_problem* prob, const void* u0, const void* targ
  * an5d_batch_create: forward only.  dA[i] holds both buffers of instance i
  * (reference layout); after a run buffer T_i%2 holds u_T, bit for bit the
  * single-grid result.  cfgs (optional): per-instance bt (<= 5; 0: the
- * depth of least cost for the instance's tiles, 5 on streams) and sl (the
+ * depth of least cost for the instance's tiles or streams) and sl (the
  * streams' segment length, 0: batch-wide; tiles have no segments).
  *
  * an5d_batch_adjoint_create: forward + adjoint.  Currently switched off: it

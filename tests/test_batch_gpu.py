@@ -312,7 +312,7 @@ def test_large_batch_on_streams(torch_cuda):
     units = 0
     for (name, n, T, _) in specs:
         r = O.info(name)["rad"]
-        for k in pyan5d.schedule(T, 5):
+        for k in pyan5d.schedule(T, {9: 3, 6: 3, 7: 3, 5: 5, 0: 5}[T]):  # the schedules of least cost
             units += -(-n[1] // (256 - 2 * k * r)) * -(-n[0] // min(64, n[0]))
     assert b.units == units
     for rep in range(3):
