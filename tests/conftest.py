@@ -22,3 +22,15 @@ def torch_cuda():
     if not torch.cuda.is_available():
         pytest.fail("torch sees no GPU in this process")
     return torch
+
+
+@pytest.fixture(autouse=True, scope="module")
+def packaged_table():
+    """Modules that clear or replace the autotuner's table leave the library's
+    own one to the modules after them: calls without a configuration are tested
+    as callers make them."""
+    yield
+    pyan5d = sys.modules.get("pyan5d")
+    if pyan5d is not None:
+        pyan5d.tune_clear()
+        pyan5d.tune_load()

@@ -664,17 +664,27 @@ def test_register_tiles_in_fma_mode(name, dt):
                 assert np.max(np.abs(got - ref)) <= tol
 
 
-def test_box3d_rows_shorter_than_a_run_beside_a_row_of_columns():
+def test_box3d_rows_shorter_than_a_run_beside_a_row_of_columns(tmp_path):
     """A grid whose nearest table row names the column kernel, but whose rows are
     shorter than a lane's run: the default path takes the direct kernel, one cell
     more the columns."""
     name, T = "box3d2r", 2
-    for n, kind in (([500, 600, 3], 1), ([500, 600, 4], 4)):
-        c = pyan5d.resolve_config(name, n, np.float64)
-        print("case columns beside a row", name, n, c, flush=True)
-        assert pyan5d.variants(name, 1)[c["variant"]]["kind"] == kind
-        A = rand_grid(name, n, np.float64, seed=5)
-        B = A.copy()
-        pyan5d.forward_host(name, A, n, T)
-        O.run(name, B, n, T)
-        assert same(A[T % 2], B[T % 2])
+    vs = pyan5d.variants(name, 1)
+    cols, = [v["index"] for v in vs if v["kind"] == 4]
+    path = tmp_path / "t.tsv"
+    path.write_text(f"{name} 1 0 96 96 96 {cols} 1 4 1.0\n")
+    pyan5d.tune_clear()
+    pyan5d.tune_load(str(path))
+    try:
+        for n, kind in (([500, 600, 3], 1), ([500, 600, 4], 4)):
+            c = pyan5d.resolve_config(name, n, np.float64)
+            print("case columns beside a row", name, n, c, flush=True)
+            assert vs[c["variant"]]["kind"] == kind
+            A = rand_grid(name, n, np.float64, seed=5)
+            B = A.copy()
+            pyan5d.forward_host(name, A, n, T)
+            O.run(name, B, n, T)
+            assert same(A[T % 2], B[T % 2])
+    finally:
+        pyan5d.tune_clear()
+        pyan5d.tune_load()
