@@ -498,37 +498,44 @@ int stream_bt(const Inst& I) {
   return best;
 }
 
-// Streams for a forward batch whose levels fill the chip with them, where they do
-// less work per cell than register tiles.  ns per 1000 cell-steps, streams at five
-// steps a launch / tiles at their own depth, 400 M and 138 M cells in a level:
-//   j2d5pt over 118 0.54/0.72, 0.66/0.73; over 7 0.74/0.95; undivided 0.74/0.59
-//   j2d9pt over 118 0.87/1.21, 0.92/1.22; over 7 1.17/1.45; undivided 1.17/1.08
-//   j2d9pt-gol over 118 0.77/0.99, 0.83/1.00; undivided 1.02/0.83
-//   star2d2r 0.64/1.06, 0.69/1.07; over 7 1.03/1.34
-// with fewer cells the streams take about 16 / (M cells) more (64 M: 0.80/0.75,
-// 1.15/1.28, 1.09/1.02 and 0.90/1.07 in the same order), so the line lies at
-// 100 M, for the two stencils of nine points and a divisor at 200 M (at three steps,
-// 138 M: 1.24/1.22 and 1.13/1.10).  At a caller's three steps streams are also
-// ahead undivided (0.79/0.95, 1.10/1.21, 0.97/1.08), at one and two the tiles are
-// (2.4/3.2, 1.4/1.7).
+// What a cell-step costs on either kernel of a forward batch whose levels fill the
+// chip, ns per 1000: one stencil, 400 M cells in a level, streams at five steps a
+// launch and tiles at their own depth, or both at a caller's three.  [kind of
+// kBatchIds][undivided, any divisor, the source's]
+struct LevelCost {
+  double stream, tile;
+};
+constexpr LevelCost kDeepCost[kBatchKinds][3] = {{{0.74, 0.59}, {0.74, 0.95}, {0.54, 0.72}},
+                                                 {{1.17, 1.08}, {1.17, 1.45}, {0.87, 1.21}},
+                                                 {{0.64, 1.05}, {1.03, 1.34}, {1.03, 1.34}},
+                                                 {{1.02, 0.83}, {1.02, 1.17}, {0.77, 0.99}}};
+constexpr LevelCost kThreeCost[kBatchKinds][3] = {{{0.79, 0.95}, {0.80, 1.01}, {0.73, 0.98}},
+                                                  {{1.10, 1.21}, {1.10, 1.35}, {0.94, 1.22}},
+                                                  {{0.82, 1.19}, {1.10, 1.28}, {1.10, 1.28}},
+                                                  {{0.97, 1.08}, {0.97, 1.15}, {0.80, 1.11}}};
+constexpr LevelCost kTwoCost{1.65, 1.5}, kOneCost{3.2, 2.5};  // bound by memory: the same for all
+
+// Streams for a forward batch where they cost less.  Levels of fewer cells leave
+// SIMDs to their warm-up planes and tails: 18 / (M cells) ns more (j2d5pt over 118,
+// streams: 0.66 at 138 M, 0.80 at 64 M, 1.51 at 15 M, where the tiles stay at 0.73
+// to 0.85).  24 mixed grids of 256^2 .. 4096^2 (25 M cells in a level) take 18 ms on
+// tiles and 45 on streams, 96 of them (100 M) 101 and 113.
 bool prefer_streams(const an5d_batch* b) {
   auto work = [](const Inst& I) { return (double)(I.g.D0 - 2 * I.g.r) * (I.g.D2 - 2 * I.g.r) * I.T; };
-  double total = 0, favoured = 0;
+  double total = 0, gain = 0;
   int longest = 0;
   for (const Inst& I : b->inst) {
+    const int form = I.has_div == 0 ? 0 : (I.has_div == 2 ? 2 : 1);
+    const LevelCost c = I.bt_fixed == 1   ? kOneCost
+                        : I.bt_fixed == 2 ? kTwoCost
+                        : I.bt_fixed == 3 ? kThreeCost[I.kind][form]
+                                          : kDeepCost[I.kind][form];
     total += work(I);
+    gain += work(I) * (c.tile - c.stream);
     if (I.T > longest) longest = I.T;
   }
-  if (longest == 0) return false;
-  const double cells = total / longest;  // of a level, on average
-  for (const Inst& I : b->inst) {
-    const StencilRT& s = stencil_rt(I.stencil);
-    const bool star2 = s.rad == 2 && s.divisor == 0;
-    if (I.bt_fixed != 0 && I.bt_fixed < 3) continue;
-    if (!I.has_div && !star2 && I.bt_fixed != 3) continue;
-    if (cells >= (star2 || s.ntaps <= 5 ? 100e6 : 200e6)) favoured += work(I);
-  }
-  return 2 * favoured > total;
+  // 18 / (cells of a level in M) on every cell-step
+  return longest > 0 && gain > 18e6 * longest;
 }
 
 // Forward batch: every instance's launch schedule under the batch's bt
