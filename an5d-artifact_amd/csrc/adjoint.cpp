@@ -237,12 +237,15 @@ __global__ __launch_bounds__(256) void adj_finish_kernel(const double* __restric
 // stream runs its sl planes, its warm-up and what fills whole ring lengths; a
 // tile runs its rows once, but extends and exchanges them anew at every step,
 // which costs kTileCost stream cells per cell (fitted, by radius and shape).
-// Forward + adjoint of 60 steps, streamed / small tile / large tile, us:
-//   j2d5pt      256^2 352/208/224  1024^2 557/584/425  2048^2 1417/1904/1338
-//   j2d9pt      256^2 569/546/465  1024^2 874/1050/916  2048^2 1806/3155/2654
-//   j2d9pt-gol  256^2 436/305/293  1024^2 715/943/595  2048^2 1436/2812/1706
-//   star2d4r    256^2 1423/1040    1024^2 1717/2369
-//   box2d2r     512^2 1187/-/784   1024^2 2199/-/1476   2048^2 4327/-/5334
+// Forward + adjoint of 40 steps, streams / 16 waves / 8 waves, us (-: not built, or
+// no streams timed):
+//   star2d1r    512^2 -/167/171   1000^2 384/410/303   2000^2 705/1220/841
+//   j2d5pt      2000^2 713/1239/861   1000x4000 714/1239/861
+//   j2d9pt      512^2 405/-/341   1000^2 572/-/580
+//   j2d9pt-gol  512^2 -/232/219   1000^2 -/520/395
+//   box2d2r     512^2 815/-/550   1000^2 1196/-/991   2000^2 2416/-/2777
+// and of radius 3-4, streams / 8 waves: star2d3r 512^2 813/650, 1000^2 990/1068;
+// star2d4r 512^2 991/734, 700^2 1030/1118.
 // With `slots` the call also counts the gradient slots any choice may need.
 static int adj_launch_plan(const AdjPlan& ap, int k, AdjLaunch& l, dim3& grid, dim3& block, AdjFn& fn,
                            long long* slots) {

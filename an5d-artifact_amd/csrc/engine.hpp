@@ -34,8 +34,8 @@ inline hipError_t lds_opt_in(const void* kernel, size_t lds, std::atomic<int>* d
 // kRows: one step per launch, rows streamed with per-row partial sums (2D
 // boxes); launched with a one-step sweep's layout
 // kCols: one step per launch, a column (3D) or run (2D) of cells per lane, for
-// the boxes of radius >= 2; in 3D its coefficient table has an order of its own
-// (cols_coefs)
+// the boxes of radius >= 2 and the 27-point boxes; at radius >= 2 in 3D its
+// coefficient table has an order of its own (cols_coefs)
 // kTile: several steps per launch on a tile held in registers
 enum KernelKind { kSweep = 0, kDirect = 1, kPlane = 2, kRows = 3, kCols = 4, kTile = 5 };
 enum DType { kF32 = 0, kF64 = 1 };

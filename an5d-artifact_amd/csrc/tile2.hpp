@@ -10,12 +10,15 @@
 // that is not the grid's own edge, so the number of steps is a trade of halo
 // against launches; it is a run-time value, one kernel serves every depth.
 // Waves whose rows are all given up stop computing and only keep the barriers.
-// Bound by launch latency and barriers up to about 512^2, by vector issue above
-// (a tile of 128 x 64 computes 1.3-2 cells per stored one).  Measured, one step,
+// Bound by launch latency, barriers and a lone wave's LDS round trips up to about
+// 512^2 (256^2: the vector units issue a fifth of the time), by vector issue and
+// those phases together above (FMA 1000x3001: they issue half of it; a tile of 128 x
+// 64 computes 1.3-2 cells per stored one).  Measured, one step,
 // best streamed configuration -> tile: j2d5pt FP32 256^2 1.43 -> 0.62 us, 512^2
 // 1.73 -> 0.98, 1024^2 2.69 -> 1.80; star2d2r FP32 1024^2 5.97 -> 1.92, 4096^2
 // 18.2 -> 14.5; star2d4r FP32 1024^2 10.2 -> 4.9; gradient2d FP64 2048^2 14.7 ->
-// 10.6.  From 4096^2 on the streams of the radius-1 stencils win.
+// 10.6.  The streams win from about 6144^2 (star2d1r, box2d1r FP32) to 8192^2 on
+// (j2d5pt FP32), sooner at radius 2 and more.
 // Shapes (tile2_inst.hip): 64 x 32 cells (few per lane, most workgroups) for the
 // smallest grids, 128 x 64 on 16 or 8 waves above; radius 3-4 needs four cells
 // a lane (256 wide).  FP32 also has 128 x 128 on 16 waves, which computes 1.2-1.5

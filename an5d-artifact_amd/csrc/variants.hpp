@@ -63,7 +63,7 @@ constexpr Shape sweep_shape(int which) {
       return Shape{0, 0, 0, 0};
     }
     if constexpr (R == 2) {
-      if (is_box<D>()) return Shape{0, 0, 0, 0};  // direct kernel only
+      if (is_box<D>()) return Shape{0, 0, 0, 0};  // column and direct kernels only
       if (which == 0) return Shape{2, 4, 8, 3};
       if (which == 1 && !f64) return Shape{3, 4, 8, 2};
       return Shape{0, 0, 0, 0};

@@ -52,7 +52,9 @@ typedef struct an5d_problem {
 
 /* Tiling.  bt: timesteps fused per launch (0: tuned/default).  variant:
  * index into an5d_variant_info() for this stencil x dtype (-1: tuned or
- * default).  sl: planes per streaming segment along dim 0 (0: default).
+ * default).  sl: planes per streaming segment along dim 0 (0: default; the
+ * register tiles, kind 5, and the direct kernel, kind 1, have no segments, so
+ * it has no effect where they are chosen).
  * mode: AN5D_EXACT (0) reproduces the C loop bit for bit (source term order,
  * no contraction, correctly rounded division); AN5D_FAST (1) folds the
  * divisor into the coefficients and chains FMAs (results within the
@@ -89,7 +91,11 @@ typedef struct an5d_variant_info {
                recomputed (3D stars of radius 2-4: the plane staged in LDS;
                3D radius-1 boxes: plane-streamed partial sums), 3: one step
                per launch, row-streamed partial sums (2D boxes of radius
-               2-4) */
+               2-4), 4: one step per launch, columns or runs of cells per
+               lane with partial sums (the 3D boxes, the 2D boxes of radius
+               2-4), 5: several steps per launch on a tile held in registers
+               (2D stars, gradient2d, the 2D boxes of radius 1-2, the
+               radius-1 3D stencils) */
   int ck, cj, nw, btmax;
   long long lds_bytes;
   int regcap; /* registers per lane the compiler was held to in the deeper
